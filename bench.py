@@ -740,6 +740,11 @@ def main():
     itemsize = 4 if solver.dtype == np.single else 8
     npml = pml_nodes(shape, pads)
     b_fwd, b_adj = algorithmic_bytes([(npts, npml)] * len(shots), itemsize)
+    resident = problem.batch.resident_tables()
+    if resident is not None:
+        # the fields stay on the chip: a step moves the dWaveOp history alone
+        b_fwd = b_adj = npts * len(shots) * itemsize
+        traffic = {}
     ach_adj = b_adj / (adj_ms * 1e-3) / 1e9
     ach_fwd = b_fwd / (fwd_ms * 1e-3) / 1e9
     grad_bytes = nt * (b_fwd + b_adj)
@@ -781,6 +786,15 @@ def main():
                       f"256 MB Infinity Cache"),
         "misfit": float(loss.detach()), "grad_norm": gnorm,
     }
+
+    if resident is not None:
+        result["roofline"].update(bound="vector instructions of the PML rows",
+                                  kernel="k_resident2d<float,4,4> (adjoint + imaging, fields on the chip; per step)")
+        result["forward_kernel"]["kernel"] = "k_resident2d<float,4,1> (forward + dWaveOp store, fields on the chip; " \
+                                             "per step)"
+        result["residency"] = (f"LDS and registers: the shots' fields, {len(resident.group_lds)} groups of shots, "
+                               f"{resident.n_strips} strips; HBM: the dWaveOp store "
+                               f"({segment * problem.batch.total_n * 4 / 2**30:.1f} GiB)")
 
     if args.ckpt_budget_gb and not (args.profile_run or args.pmc_run):
         # the same gradient with the dWaveOp history checkpointed: the budget

@@ -346,6 +346,64 @@ int pysit_amd_plan_stats(const pysit_amd_plan *plan, long long *stats);
 /* Waits for the device, then frees the plan's graphs, cursor and stream. */
 int pysit_amd_plan_destroy(pysit_amd_plan *plan);
 
+/* ------------------------------------------------------------------------ */
+/* The 2D time loop with the wavefield held on the chip.                     */
+/*                                                                           */
+/* The same run as pysit_amd_batch_run (modes 0 to 3, no field store and no  */
+/* second-order terms; an FP32 adjoint through the FP32 window, an FP64 one  */
+/* in FP64), bit for bit, as a few launches of many steps each: a shot is    */
+/* cut along x into strips of whole rows, one workgroup per strip keeps its  */
+/* fields in registers and LDS, and neighbouring strips exchange their       */
+/* border rows through `xchg` (the reference steps its loop from Python, one */
+/* step call per time level: temporal_modeling.py:120-142, :313-350).        */
+/* Shots run in groups of at most one strip per compute unit.  The tables    */
+/* are built on the host (pysit_amd/resident.py).  A launch is cooperative:  */
+/* not for streams under capture.  The waits for a neighbour are bounded;    */
+/* one that reaches the bound (`spin` polls of about 1 us) ends the launch,  */
+/* leaves NaN in the state and writes 1 to *err, which the caller checks     */
+/* once the stream has been waited for.                                      */
+/* ------------------------------------------------------------------------ */
+typedef struct {
+    int n_strips, n_groups;
+    const int *group_begin;  /* HOST, n_groups + 1: first strip of each group   */
+    const int *group_lds;    /* HOST: LDS bytes per workgroup of each group     */
+    /* device tables: 32 ints per strip (csrc/resident2d.hip reads them as d[]);
+     * per kind of strip and thread (512) an item {row of march step 0, flags,
+     * own rows | first step << 16 | late << 24, cell column |
+     * thread whose cells it repeats << 16}; per strip with
+     * forward [0] or adjoint [1] sources and thread {first source cell, march
+     * steps with sources}; source nodes and receiver nodes in strip order   */
+    const int *strips;
+    const int *items;
+    const int *finfo[2];
+    const int *inj_lds[2], *inj_nptr[2], *inj_chan[2], *inj_shot[2];
+    const double *inj_w[2];
+    int n_inj[2];
+    const int *rec_lds;
+    int n_rec_nodes;
+    const int *rec_node;     /* node of every receiver entry (rec_w's order)    */
+    void *pre;               /* source values of pre_slots slots                */
+    int pre_slots;
+    void *recbuf;            /* receiver node values of rec_slots slots         */
+    int rec_slots;
+    void *xchg;              /* zero before the first run                       */
+    long long xchg_stride;   /* bytes per strip: 2 x 64 tags, 4 x xchg_cells    */
+    int xchg_cells;          /* cells of 16 bytes, at most, of one border       */
+    int spin;
+    int *err;                /* host memory the device can write                */
+    unsigned *epoch;         /* HOST: next step tag, 0 before the first run     */
+} pysit_amd_resident;
+
+/* What the tables must assume, limits[5]: rows of a thread's cell column
+ * (plain nodes, PML nodes), threads per workgroup, border jobs (64 columns
+ * each) per exchange wave, and per side of a strip. */
+int pysit_amd_resident_limits(int *limits);
+
+/* pysit_amd_batch_run's arguments with the resident tables; `record`: sample
+ * the receivers (modes 0, 1 and 3). */
+int pysit_amd_resident_run(const pysit_amd_batch *b, const pysit_amd_resident *r, int mode, int slot_begin,
+                           int slot_end, int direction, int seg_base, int record, void *stream);
+
 /* Sum of squares over time slots of a slot-major store (the dWaveOp store):
  * out[i] += sum over s = slot_begin, slot_begin + slot_step, ... < slot_end of
  * store[s * slot_stride + i]^2 in FP64, for i < n (store: dtype 0 f32 or

@@ -55,6 +55,20 @@ class Batch(ctypes.Structure):
     ]
 
 
+class Resident(ctypes.Structure):
+    """``pysit_amd_resident``."""
+    _fields_ = [
+        ("n_strips", _i), ("n_groups", _i), ("group_begin", _vp), ("group_lds", _vp),
+        ("strips", _vp), ("items", _vp), ("finfo", _vp * 2),
+        ("inj_lds", _vp * 2), ("inj_nptr", _vp * 2), ("inj_chan", _vp * 2), ("inj_shot", _vp * 2),
+        ("inj_w", _vp * 2), ("n_inj", _i * 2),
+        ("rec_lds", _vp), ("n_rec_nodes", _i), ("rec_node", _vp),
+        ("pre", _vp), ("pre_slots", _i), ("recbuf", _vp), ("rec_slots", _i),
+        ("xchg", _vp), ("xchg_stride", _ll), ("xchg_cells", _i), ("spin", _i),
+        ("err", _vp), ("epoch", _vp),
+    ]
+
+
 class NativeError(RuntimeError):
     pass
 
@@ -75,6 +89,8 @@ SIGNATURES = {
     "pysit_amd_batch_run": [ctypes.POINTER(Batch), _i, _i, _i, _i, _i, _vp, _vp, _vp],
     "pysit_amd_batch_run_static": [ctypes.POINTER(Batch), _i, _i, _i, _i, _i, _vp, _vp, _vp],
     "pysit_amd_batch_run_persistent": [ctypes.POINTER(Batch), _i, _i, _i, _i, _i, _vp, _vp, _vp],
+    "pysit_amd_resident_limits": [_vp],
+    "pysit_amd_resident_run": [ctypes.POINTER(Batch), ctypes.POINTER(Resident), _i, _i, _i, _i, _i, _i, _vp],
     "pysit_amd_fold": [_i] * 10 + [_vp, _d, _vp, _i, _i, _i, _vp],
     "pysit_amd_slot_square_sum": [_vp, _i, _ll, _i, _i, _i, _ll, _vp, _vp],
     "pysit_amd_plan_create": [_i, _i, ctypes.POINTER(_vp)],
@@ -121,6 +137,14 @@ def tile_rows_supported(dim, dtype_code, tile_x):
     if n < 0:
         raise NativeError(lib().pysit_amd_last_error().decode())
     return n == 1
+
+
+def resident_limits():
+    """(plain rows, PML rows of a thread's column, threads per workgroup,
+    border operations per exchange wave and per side) of the resident loop."""
+    v = (_i * 5)()
+    call("pysit_amd_resident_limits", ctypes.cast(v, _vp))
+    return tuple(v)
 
 
 def call(name, *args):

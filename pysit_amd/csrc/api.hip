@@ -22,6 +22,10 @@ template <typename T>
 int run2d_persistent(const pysit_amd_batch &, int, int, int, int, int, const int *, const int *, long long,
                      hipStream_t);
 
+template <typename T>
+int run2d_resident(const pysit_amd_batch &, const pysit_amd_resident &, int, int, int, int, int, int, hipStream_t);
+void resident_rows(int *plain, int *full, int *threads, int *ops, int *tags);
+
 int ic_flush(const pysit_amd_batch &B, hipStream_t st);
 int tile_rows_2d(int dtype);
 bool tile_rows_2d_supported(int tx);
@@ -171,7 +175,7 @@ __global__ void k_slot_square_sum(const T *__restrict__ store, long long stride,
     out[i] += acc;
 }
 
-static int inj_precompute(const pysit_amd_batch &B, int slot_begin, int slot_end, int seg_base, hipStream_t st)
+int inj_precompute(const pysit_amd_batch &B, int slot_begin, int slot_end, int seg_base, hipStream_t st)
 {
     if (slot_end <= slot_begin || B.n_inj_nodes == 0) return PYSIT_AMD_OK;
     const dim3 grid((unsigned)((B.n_inj_nodes + 255) / 256),
@@ -293,13 +297,10 @@ int pysit_amd_cda_step3d_f64(int order, const double *km1_u, const double *k_phi
 
 namespace pa {
 
-// pysit_amd_batch_run's checks and dispatch, with an optional plan
-static int batch_run(const pysit_amd_batch *b, int mode, int slot_begin, int slot_end, int direction,
-                     int seg_base, const int *active_tiles, const int *active_recs, pysit_amd_plan *plan,
-                     void *stream, long long persistent_spins = 0)
+// the checks of a run's arguments
+static int check_run(const pysit_amd_batch &B, int mode, int slot_begin, int slot_end, int direction, int seg_base,
+                     const int *active_tiles, const int *active_recs)
 {
-    PA_CHECK(b != nullptr, "null batch");
-    const pysit_amd_batch &B = *b;
     PA_CHECK(B.dim == 2 || B.dim == 3, "dim must be 2 or 3");
     PA_CHECK(B.dtype == 0 || B.dtype == 1, "dtype must be 0 (f32) or 1 (f64)");
     PA_CHECK(B.order == 2 || B.order == 4 || B.order == 6 || B.order == 8,
@@ -340,6 +341,18 @@ static int batch_run(const pysit_amd_batch *b, int mode, int slot_begin, int slo
                      "active receiver count out of range");
         }
     }
+    return PYSIT_AMD_OK;
+}
+
+// pysit_amd_batch_run's checks and dispatch, with an optional plan
+static int batch_run(const pysit_amd_batch *b, int mode, int slot_begin, int slot_end, int direction,
+                     int seg_base, const int *active_tiles, const int *active_recs, pysit_amd_plan *plan,
+                     void *stream, long long persistent_spins = 0)
+{
+    PA_CHECK(b != nullptr, "null batch");
+    const pysit_amd_batch &B = *b;
+    const int bad = check_run(B, mode, slot_begin, slot_end, direction, seg_base, active_tiles, active_recs);
+    if (bad) return bad;
     PA_CHECK(!B.inj_pre || (B.inj_ptr && B.inj_node_shot && B.n_inj_nodes >= 0 && B.inj_pre_slots >= 0 &&
                             slot_end - seg_base <= B.inj_pre_slots &&
                             (slot_end - slot_begin + kInjPreSlots - 1) / kInjPreSlots <= 65535),
@@ -490,6 +503,35 @@ int pysit_amd_plan_run(pysit_amd_plan *plan, const pysit_amd_batch *b, int mode,
     PA_CHECK(dev == plan_device(plan), "the plan belongs to another device");
     return batch_run(b, mode, slot_begin, slot_end, direction, seg_base, active_tiles, active_recs, plan,
                      stream);
+}
+
+int pysit_amd_resident_limits(int *limits)
+{
+    clear_error();
+    PA_CHECK(limits, "null argument");
+    resident_rows(limits, limits + 1, limits + 2, limits + 3, limits + 4);
+    return PYSIT_AMD_OK;
+}
+
+int pysit_amd_resident_run(const pysit_amd_batch *b, const pysit_amd_resident *r, int mode, int slot_begin,
+                           int slot_end, int direction, int seg_base, int record, void *stream)
+{
+    clear_error();
+    PA_CHECK(b && r, "null argument");
+    const pysit_amd_batch &B = *b;
+    const int bad = check_run(B, mode, slot_begin, slot_end, direction, seg_base, nullptr, nullptr);
+    if (bad) return bad;
+    PA_CHECK(B.dim == 2, "the resident loop is built for 2D batches");
+    PA_CHECK(!B.fstore && !B.dw_out && !B.vol_dw, "the resident loop stores no field and has no second-order terms");
+    PA_CHECK(mode == 2 ? direction == -1 : direction == 1, "the resident loop runs forward, its adjoint backward");
+    PA_CHECK(r->n_groups >= 1 && r->group_begin && r->group_lds && r->strips && r->items && r->finfo[0] &&
+                 r->xchg && r->err && r->epoch && r->spin >= 1,
+             "resident tables missing");
+    if (slot_end <= slot_begin) return PYSIT_AMD_OK;
+    return B.dtype ? run2d_resident<double>(B, *r, mode, slot_begin, slot_end, direction, seg_base, record,
+                                            (hipStream_t)stream)
+                   : run2d_resident<float>(B, *r, mode, slot_begin, slot_end, direction, seg_base, record,
+                                           (hipStream_t)stream);
 }
 
 int pysit_amd_slot_square_sum(const void *store, int dtype, long long slot_stride, int slot_begin, int slot_end,

@@ -26,6 +26,7 @@ import numpy as np
 import torch
 
 from . import _native as N
+from .resident import ResidentTables
 
 TILE_Z = 64      # z nodes per wavefront (the contiguous axis)
 
@@ -244,6 +245,9 @@ GRAPH_MAX_NODES = 1 << 20
 # default graph chunk, a multiple of it so that graph chunks hold whole windows
 IC_WINDOW = 64
 GRAPH_STEPS = 64
+# shorter runs than this many slots go through the step kernels: a resident
+# launch loads and stores the whole state
+RESIDENT_MIN_SLOTS = 8
 
 
 class DeviceBatch:
@@ -255,7 +259,7 @@ class DeviceBatch:
 
     def __init__(self, shots, model, deltas, dt, order, dtype=np.float32, tile_x=None,
                  imaging_period=1, memory_budget=None, ic_window=None, tile_order="shot", graph_steps=None,
-                 adjoint="pysit"):
+                 adjoint="pysit", resident=None):
         if not shots:
             raise ValueError("empty shot batch")
         self.dim = shots[0].dim
@@ -332,6 +336,15 @@ class DeviceBatch:
         # device-wide barrier between steps costs more than a graph's launch
         # boundary on MI355X, hence off by default.
         self.persistent = False
+
+        # 2D time loops with the wavefield held on the chip (resident.py): on
+        # unless a launch configuration of the step kernels is asked for
+        # (tile_x, tile_order, graph_steps) or the batch does not suit it;
+        # True: also where the step kernels are expected to be faster
+        self._resident_always = resident is True
+        if resident is None:
+            resident = not tile_x and graph_steps is None and tile_order == "shot"
+        self._resident = None if resident else False  # False: never; None: tables not built yet
 
         if isinstance(model, torch.Tensor):
             self.model = model.detach().to(device=self.dev, dtype=self.tdtype).contiguous()
@@ -491,6 +504,7 @@ class DeviceBatch:
 
         # receivers
         recs, ridx, rw = [], [], []
+        self._rec_sorted = []  # per shot, the entries' flat padded nodes in rec_w's order
         e = 0
         for si, s in enumerate(self.shots):
             idx, chan, w = s.rec
@@ -498,6 +512,7 @@ class DeviceBatch:
             idx = (np.asarray(idx, dtype=np.int64) // nz) * self.zs[si] + np.asarray(idx, dtype=np.int64) % nz
             order = np.argsort(chan, kind="stable")
             idx, chan, w = idx[order], chan[order], w[order]
+            self._rec_sorted.append((idx // self.zs[si]) * nz + idx % self.zs[si])
             counts = np.bincount(chan, minlength=s.nrec)
             starts = np.concatenate([[0], np.cumsum(counts)])
             for r in range(s.nrec):
@@ -815,6 +830,29 @@ class DeviceBatch:
         b.imaging_period = self.imaging_period
         return b
 
+    def resident_tables(self):
+        """The tables of the resident loop, or None if this batch does not
+        use it."""
+        if self._resident is None:
+            self._resident = ResidentTables.build(self, self._resident_always) or False
+        return self._resident or None
+
+    def _resident_for(self, b, mode, slots):
+        """The resident tables if a run of ``slots`` slots goes through them:
+        not the runs with a field store or second-order terms, an adjoint
+        without imaging or with the other accumulator, short runs (a launch
+        loads and stores the whole state) and streams under capture (the
+        launch is cooperative)."""
+        if (slots < RESIDENT_MIN_SLOTS or b.fstore or b.dw_out or b.vol_dw or self.persistent
+                or not self.precompute_injection):
+            return None
+        if mode == 2 and (not b.dw or bool(b.ic32) != (self.dtype == np.float32)):
+            return None
+        tables = self.resident_tables()
+        if tables is None or torch.cuda.is_current_stream_capturing():
+            return None
+        return tables
+
     def _run(self, b, mode, j0, j1, direction, seg_base, record=True):
         at = np.ascontiguousarray(self.active_tiles)
         ar = np.ascontiguousarray(self.active_recs if record else np.zeros_like(self.active_recs))
@@ -823,7 +861,10 @@ class DeviceBatch:
             ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
             ev[0].record()
         atp, arp = at.ctypes.data_as(ctypes.c_void_p), ar.ctypes.data_as(ctypes.c_void_p)
-        if (self.persistent and self.dim == 2 and mode in (0, 1, 2) and not (b.dw_out or b.vol_dw)
+        resident = self._resident_for(b, mode, j1 - j0)
+        if resident is not None:
+            resident.run(self, b, mode, j0, j1, direction, seg_base, record, _stream())
+        elif (self.persistent and self.dim == 2 and mode in (0, 1, 2) and not (b.dw_out or b.vol_dw)
                 and self.tile_x in (8, 4)):
             N.call("pysit_amd_batch_run_persistent", ctypes.byref(b), mode, j0, j1, direction, seg_base, atp, arp,
                    _stream())
@@ -1174,7 +1215,10 @@ class DeviceBatch:
         # segment) are evaluated before its first step: a step then reads one
         # value per node instead of gathering the node's receiver entries
         n_nodes = int(self.adj_inj[2].numel()) - 1
-        if n_nodes > 0 and self.precompute_injection:
+        # (the resident loop evaluates them itself, a chunk of slots at a time)
+        held = image and not (second or store_field or binomial) and self.dim == 2 and not self.persistent \
+            and (self.dtype == np.float64) != (ic32 is not None) and self.resident_tables() is not None
+        if n_nodes > 0 and self.precompute_injection and not held:
             slots = K if ((self.ckpts or binomial) and image) else self.max_nt
             qb.inj_pre = self._inj_pre_buffer(slots, n_nodes).data_ptr()
             qb.inj_node_shot = self.adj_inj[5].data_ptr()

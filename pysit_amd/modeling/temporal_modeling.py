@@ -155,6 +155,11 @@ class TemporalModeling(object):
         kw = dict(dtype=s.dtype, imaging_period=imaging_period, memory_budget=self.memory_budget,
                   ic_window=self.ic_window, adjoint=self.adjoint)
         if self.autotune and not self.tile_x:
+            if s.mesh.dim == 2:
+                b = DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
+                if b.resident_tables() is not None:
+                    return b  # its loop has no launch configuration to tune
+                del b
             from ..autotune import tuned_batch
             return tuned_batch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
         return DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, tile_x=self.tile_x,

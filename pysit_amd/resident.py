@@ -1,0 +1,649 @@
+"""Host tables of the 2D time loop that keeps the wavefield on the chip
+(``pysit_amd_resident_run``, csrc/resident2d.hip).
+
+A shot is cut along x into strips of whole rows, one workgroup each; a
+workgroup's threads own 16-byte cell columns (4 FP32 or 2 FP64 nodes along z)
+over a few rows.  Cells away from the PML and the grid's edges take the plain
+update (their waves are *plain*), the others the PML update (*full*).  Shots
+that do not fit the GPU together run one group after the other.
+
+Everything here is numpy on the host; :class:`ResidentTables` uploads the
+result once per batch geometry.
+"""
+import ctypes
+
+import numpy as np
+
+from . import _native as N
+
+# LDS a workgroup may use
+LDS_BYTES = 160 * 1024
+STRIP_INTS = 32
+REV, BEGIN_TOP, BEGIN_BOT, KIND, END_TOP, END_BOT = 1, 2, 4, 8, 32, 64
+XTYPE, PXTOP, PXBOT = 1, 2, 4
+# cost model of a step, in plain rows of a thread (about 600 cycles): a PML
+# row, the exchange wave's own work and the factor of the work beside it (a
+# border that is late holds up the neighbours too), what a step spends around
+# its rows, and the part of the workgroup's whole work that adds to its longest
+# SIMD's.  Fitted to the step times of 11 batches: 77 x 67 to 1041 x 341, FP32
+# and FP64, 1 to 32 shots; models with the wait for a neighbour as a cost of
+# its own chose fewer, higher strips for few shots, up to 1.5 times slower.
+FULL_COST = 6.0
+EXCHANGE_COST = 1.5
+EXCHANGE_SHARE = 1.5
+STEP_COST = 2.0
+SHARE_COST = 1.0
+# what a step of the step kernels costs, in the same unit: launch and latency,
+# and the bytes of one field that add 1
+STEP_KERNEL_COST = 35.0
+STEP_KERNEL_BYTES = 30000.0
+# device memory for the source values and receiver nodes of a chunk of slots
+CHUNK_BYTES = 256 << 20
+SPIN = 1 << 20
+
+
+def z_columns(nz, nzl, nzr, R, V):
+    """(cells of a row, full cells at the left, full cells at the right): a
+    cell is full if a node within R of it is a PML node, an edge node or
+    beyond the grid."""
+    nzc = -(-nz // V)
+    fl = min(nzc, -(-(max(nzl, 1) + R) // V))
+    # the first cell whose last node reaches the right band
+    first = max(0, -(-(nz - max(nzr, 1) - R - (V - 1)) // V))
+    fr = max(0, nzc - first)
+    if fl + fr >= nzc:
+        return nzc, nzc, 0
+    return nzc, fl, fr
+
+
+def _groups(nr, n):
+    """n row groups (first row, rows) of nr rows, the larger ones first."""
+    base, extra = divmod(nr, n)
+    out, r = [], 0
+    for g in range(n):
+        k = base + (g < extra)
+        out.append((r, k))
+        r += k
+    return out
+
+
+class Layout(object):
+    """How the threads of one workgroup share a strip of ``nr`` rows with
+    ``plain`` and ``full`` cell columns.  The threads of a kind take row
+    groups column by column, the groups at the strip's borders first: a wave
+    with one of them waits for the neighbours' rows.  PML rows near a border
+    may be groups of one row, so that little is left to do after the wait.
+    ``waves``: per wave its kind (1 plain, 2 full, 3 exchange, 0 idle) and its
+    first thread among those of its kind; ``cost``: a step in plain rows."""
+
+    def __init__(self, nr, plain, full, limits, border, R, alone):
+        self.nr, self.plain, self.full = nr, plain, full
+        rp, rf, threads, jobs, tags = limits
+        R = 0 if alone else R  # no neighbour's rows to wait for
+        n_waves = threads // 64
+        best = None
+        plains = [(pg, self._kind_waves(1, pg, plain, 1.0, nr, R)) for pg in self._plain_groups(nr, plain, rp, n_waves)]
+        for fg in self._full_groups(nr, full, rf, n_waves, R):
+            full_waves = self._kind_waves(2, fg, full, FULL_COST, nr, R)
+            for pg, plain_waves in plains:
+                waves = full_waves + plain_waves
+                # the rest exchange the border rows, `border` jobs a side
+                ex = min(n_waves - len(waves), max(1, 2 * border))
+                if ex < 1 or border > tags or 2 * border > jobs * ex:
+                    continue
+                waves += [(EXCHANGE_COST, 0, 3, 0)] * ex
+                waves += [(0.0, 0, 0, 0)] * (n_waves - len(waves))
+                waves.sort(reverse=True)
+                waves = waves[:4] + waves[4:][::-1]  # wave w runs on SIMD w % 4
+                # waves w and w + 4 share a SIMD; a border that is late holds up
+                # the neighbours too, so work beside an exchange wave counts more
+                cost = max(a[0] * (EXCHANGE_SHARE if b[2] == 3 else 1.0) +
+                           b[0] * (EXCHANGE_SHARE if a[2] == 3 else 1.0) for a, b in zip(waves[:4], waves[4:]))
+                work = sum(w[0] for w in waves)
+                key = (cost + STEP_COST + SHARE_COST * work, work)
+                if best is None or key < best[0]:
+                    best = (key, fg, pg, ex, [(k, t) for _, _, k, t in waves])
+        self.ok = best is not None
+        if self.ok:
+            (self.cost, _), self.full_groups, self.plain_groups, self.exchange, self.waves = best
+
+    @staticmethod
+    def _counts(nr, cols, most, n_waves):
+        """Numbers of row groups of at most ``most`` rows that differ in their
+        size and fit the waves."""
+        return sorted({-(-nr // k) for k in range(1, most + 1)} - {n for n in range(nr + 1) if n * cols > 64 * (n_waves - 1)})
+
+    @classmethod
+    def _full_groups(cls, nr, full, rf, n_waves, R):
+        """Candidate splits: lists of row groups, each from a wave of its own."""
+        if not full:
+            return [[]]
+        out = [[_border_first(_groups(nr, n))] for n in cls._counts(nr, full, rf, n_waves)]
+        if R and nr > 2 * R:
+            inner = nr - 2 * R
+            for per in (1, 2):  # rows of a group at the border
+                edge = [(r, min(per, R - r)) for r in range(0, R, per)]
+                edge += [(nr - R + r, k) for r, k in edge]
+                for n in cls._counts(inner, full, rf, n_waves):
+                    out.append([edge, [(r + R, k) for r, k in _groups(inner, n)]])
+        return out
+
+    @classmethod
+    def _plain_groups(cls, nr, plain, rp, n_waves):
+        if not plain:
+            return [[]]
+        return [[_border_first(_groups(nr, n))] for n in cls._counts(nr, plain, rp, n_waves)]
+
+    @staticmethod
+    def _kind_waves(kind, parts, cols, unit, nr, R):
+        """(work, rows that wait for a border, kind, first thread) of the waves
+        that hold ``parts``, each part from a wave of its own."""
+        out, t0 = [], 0
+        for groups in parts:
+            n = len(groups) * cols
+            for w in range(-(-n // 64)):
+                mine = groups[w * 64 // cols:(min(n, w * 64 + 64) - 1) // cols + 1]
+                late = max(sum(x < R or x + R >= nr for x in range(r, r + k)) for r, k in mine)
+                out.append((max(k for _, k in mine) * unit, late, kind, t0))
+                t0 += 64
+        return out
+
+
+def _border_first(groups):
+    """The first and the last group, then the others."""
+    return groups[:1] + groups[:0:-1][:1] + groups[1:-1] if len(groups) > 2 else groups
+
+
+def lds_copies(strips, hc, R, n_fcells):
+    """Bytes of one copy of u, Phix, Phiz and the source cells of strips (an
+    array of their numbers, or one strip's)."""
+    nr, nzc, full = strips.T[2], strips.T[21], strips.T[4] + strips.T[5]
+    return (((nr + 2 * R) * (nzc + hc) + hc) * 16, (nr + 2 * R) * full * 16, (nr * (full + 2 * hc) + hc) * 16,
+            n_fcells * 16)
+
+
+def lds_offsets(copies, nr, itemsize):
+    """Where Phix, Phiz, the source cells, the x profiles and the flags begin:
+    u comes first, two copies each of all but the profiles."""
+    return np.cumsum([2 * c for c in copies] + [-(-nr * 2 * itemsize // 16) * 16], axis=0)
+
+
+def _split(total, rows, R):
+    """Row counts of equal strips of at most ``rows`` rows, each at least R."""
+    n = max(1, min(-(-total // rows), total // R if total >= R else 1))
+    base, extra = divmod(total, n)
+    return [base + (i < extra) for i in range(n)]
+
+
+_LAYOUTS = {}
+
+
+def _sorted_unique(a):
+    """np.unique with the inverse, without the sort where none is needed."""
+    if a.size == 0 or np.all(a[1:] > a[:-1]):
+        return a, np.arange(a.size)
+    u, inv = np.unique(a, return_inverse=True)
+    return u, inv.reshape(-1)
+
+
+class ShotStrips(object):
+    """The ways to cut one shot into strips of at most ``most`` rows: its
+    column split and, for a bound on the cost of a step, the strips (x0, rows,
+    x type)."""
+
+    def __init__(self, shape, pml, R, itemsize, limits, n_fcells_row, most):
+        (xl, xr), (zl, zr) = pml
+        self.nx, self.nz = shape
+        self.most = most
+        self.R, self.itemsize, self.limits = R, itemsize, limits
+        self.V = 16 // itemsize
+        self.hc = -(-R // self.V)
+        self.nzc, self.zfl, self.zfr = z_columns(self.nz, zl, zr, R, self.V)
+        left, right = max(xl, 1) + R, max(xr, 1) + R
+        self.n_fcells_row = n_fcells_row
+        if self.zfl == self.nzc or self.nx - left - right < max(R, 1):
+            # all cells full anyway, or no room between the x sides
+            self.segments = [(0, self.nx, True)]
+        else:
+            self.segments = [(0, left, True), (left, self.nx - left - right, False), (self.nx - right, right, True)]
+        self._costs = {}
+
+    def fits(self, nr, xtype):
+        fl, fr = (self.nzc, 0) if xtype else (self.zfl, self.zfr)
+        d = np.zeros(STRIP_INTS, dtype=np.int64)
+        d[[2, 4, 5, 21]] = nr, fl, fr, self.nzc
+        copies = lds_copies(d, self.hc, self.R, self.n_fcells_row * nr)
+        return lds_offsets(copies, nr, self.itemsize)[-1] + 32 <= LDS_BYTES
+
+    def layout(self, nr, xtype, alone=False):
+        full = self.nzc if xtype else self.zfl + self.zfr
+        # jobs of a border: u over all cells and Phix over the full ones, 64
+        # columns each
+        border = -(-self.nzc // 64) - (-full // 64)
+        key = (nr, self.nzc - full, full, self.limits, border, self.R, alone)
+        if key not in _LAYOUTS:
+            if len(_LAYOUTS) > 4096:
+                _LAYOUTS.clear()
+            _LAYOUTS[key] = Layout(*key)
+        return _LAYOUTS[key]
+
+    def costs(self, xtype):
+        """(rows, cost) of the strips that fit a workgroup, by rows."""
+        if xtype not in self._costs:
+            out = []
+            for nr in range(self.R, min(self.nx, self.most) + 1):
+                if not self.fits(nr, xtype):
+                    break
+                lay = self.layout(nr, xtype)
+                if lay.ok:
+                    out.append((nr, lay.cost))
+            self._costs[xtype] = out
+        return self._costs[xtype]
+
+    def cut(self, bound, rows_z=None):
+        """Strips that cost at most ``bound`` a step, or None: the fewest, but
+        those away from the x PML of about ``rows_z`` rows if that is given."""
+        if self.fits(self.nx, True) and rows_z is None:
+            lay = self.layout(self.nx, True, True)
+            if lay.ok and lay.cost <= bound:
+                return [(0, self.nx, True)]
+        out = []
+        for x0, total, xtype in self.segments:
+            ok = {nr for nr, c in self.costs(xtype) if c <= bound}
+            given = rows_z is not None and not xtype
+            for rows in ([rows_z] if given else sorted(ok, reverse=True)):
+                parts = _split(total, rows, self.R)
+                if all(nr in ok for nr in parts):
+                    break
+            else:
+                return None
+            for nr in parts:
+                out.append((x0, nr, xtype))
+                x0 += nr
+        return out
+
+    def bounds(self):
+        """The costs a strip of this shot can have."""
+        out = {c for _, _, xtype in self.segments for _, c in self.costs(xtype)}
+        if self.fits(self.nx, True) and self.layout(self.nx, True, True).ok:
+            out.add(self.layout(self.nx, True, True).cost)
+        return out
+
+
+def plan_groups(shots, cus):
+    """The cost of a step and the consecutive shots that run together with
+    their strips, a list of (shots, strip lists); None if a shot does not fit.  Of the ways to spread the
+    shots evenly over the fewest groups, or one or two more, the one whose
+    groups' steps cost least together; strips cost alike within a group."""
+    bounds = sorted(set().union(*[s.bounds() for s in set(shots)]))
+    if not bounds:
+        return None
+    cuts = {}
+
+    def cut(s, *bound):
+        if (s, bound) not in cuts:
+            cuts[(s, bound)] = s.cut(*bound)
+        return cuts[(s, bound)]
+
+    def fill(group):
+        """(bound, rows away from the x PML): the least bound whose strips fit
+        the compute units and, where units are left, the lowest strips beside
+        it.  Few may be as low as R rows; many exchange so many rows that those
+        of less than 2 R, where every row waits for both borders, are slower
+        (FP32, 1 shot: 1041 x 341 nodes of order 8, 6.6 us a step with 178
+        strips and 6.0 with 123; 186 x 113 of order 8, 4.9 with 24 and 6.0 with
+        19; 360 x 332 of order 4, 4.4 with 180 and 5.3 with 83)."""
+        def count(*bound):
+            c = [cut(shots[i], *bound) for i in group]
+            return cus + 1 if any(x is None for x in c) else sum(len(x) for x in c)
+        lo, hi = 0, len(bounds) - 1
+        if count(bounds[hi]) > cus:
+            return None
+        while lo < hi:
+            mid = (lo + hi) // 2
+            if count(bounds[mid]) <= cus:
+                hi = mid
+            else:
+                lo = mid + 1
+        n, R = count(bounds[lo]), max(shots[i].R for i in group)
+        for first, most in ((R, min(3 * cus // 4, 2 * cus // R)), (2 * R, cus)):
+            for rows in range(first, 4 * R):
+                if n < count(bounds[lo], rows) <= most:
+                    return bounds[lo], rows
+        return (bounds[lo],)
+
+    fewest = [cut(s, bounds[-1]) for s in shots]
+    if any(f is None or len(f) > cus for f in fewest):
+        return None
+    weight = [len(f) for f in fewest]
+    total = sum(weight)
+    best = None
+    first = max(1, -(-total // cus))
+    for n in range(first, len(shots) + 1):
+        groups, load = [[] for _ in range(n)], 0
+        for i, t in enumerate(weight):
+            groups[min(n - 1, int((load + t / 2) * n / total))].append(i)
+            load += t
+        groups = [g for g in groups if g]
+        got = [fill(g) for g in groups]
+        if all(b is not None for b in got) and (best is None or sum(b[0] for b in got) < best[0]):
+            best = (sum(b[0] for b in got), [(g, [cut(shots[i], *b) for i in g]) for g, b in zip(groups, got)])
+        if best is not None and n >= first + 2:
+            break
+    return best
+
+
+def thread_items(lay, xtype, nzc, zfl, zfr, R, limits):
+    """(threads, 4) item table of a workgroup, and the owner of every cell:
+    thread and march step, (rows, columns).  A lane left over in a wave repeats
+    the cells of another thread, which its item names."""
+    rp, rf, threads = limits[:3]
+    items = np.zeros((threads, 4), dtype=np.int32)
+    owner = np.full((lay.nr, nzc, 2), -1, dtype=np.int32)
+    alias = np.arange(threads)
+    full_cols = np.arange(nzc) if xtype else np.concatenate([np.arange(zfl), np.arange(nzc - zfr, nzc)])
+    plain_cols = np.setdiff1d(np.arange(nzc), full_cols)
+    for kind, cols, parts, RM in ((2, full_cols, lay.full_groups, rf), (1, plain_cols, lay.plain_groups, rp)):
+        # thread t of the kind: its wave by the wave's first thread
+        wave_of = {t0 // 64: w for w, (k, t0) in enumerate(lay.waves) if k == kind}
+        t0 = 0
+        for groups in parts:
+            row0, size = (np.array(v) for v in zip(*groups))
+            n = len(groups) * cols.size
+            t = np.arange(-(-n // 64) * 64)
+            live = t < n
+            g = np.where(live, t // cols.size, len(groups) - 1)
+            col, cnt, r0 = cols[t % cols.size], size[g], row0[g]
+            # the group at the top marches towards it, unless it holds every row
+            rev = (r0 == 0) & (cnt < lay.nr) & (cnt > 1)
+            top, bot = r0 < R, r0 + cnt - 1 + R >= lay.nr
+            # the border a march starts at is needed at once, the other at its end
+            wait = np.where(top, np.where(rev, END_TOP, BEGIN_TOP), 0) | np.where(bot, np.where(rev, BEGIN_BOT, END_BOT), 0)
+            flags = np.where(rev, REV, 0) | np.where(live, wait, 0) | KIND * kind
+            rbase = np.where(rev, r0 + RM - 1, r0 - (RM - cnt))
+            own = np.where(live, ((1 << RM) - 1) & ~((1 << (RM - cnt)) - 1), 0)
+            first = (RM - cnt).reshape(-1, 64).min(axis=1).repeat(64)
+            late = RM - cnt > first
+            tids = np.array([wave_of[t0 // 64 + i] for i in t // 64]) * 64 + t % 64
+            items[tids] = np.stack([rbase, flags, own | (first << 16) | (late.astype(np.int64) << 24), col], axis=1)
+            for j in range(RM):
+                m = ((own >> j) & 1) == 1
+                row = rbase[m] + j * np.where(rev[m], -1, 1)
+                owner[row, col[m], 0] = tids[m]
+                owner[row, col[m], 1] = j
+            alias[tids] = owner[r0, col, 0]
+            t0 += t.size
+    # the exchange waves know their number, the idle ones follow them
+    for i, w in enumerate(sorted((w for w, (k, _) in enumerate(lay.waves) if k in (0, 3)),
+                                 key=lambda w: -lay.waves[w][0])):
+        items[64 * w:64 * w + 64, 0] = i
+        items[64 * w:64 * w + 64, 1] = 3 * KIND
+    items[:, 3] |= alias << 16
+    return items, owner
+
+
+_PLANS = {}
+
+
+class Plan(object):
+    """What the sizes of a batch's shots (``keys``: shape, PML widths and most
+    source cells of a row) decide: the groups, the strips without their
+    sources and receivers, and the thread tables of the kinds of strips.
+    ``ok`` is False where a shot does not suit the loop."""
+
+    @classmethod
+    def of(cls, keys, R, itemsize, limits, cus):
+        key = (keys, R, itemsize, limits, cus)
+        plan = _PLANS.get(key)
+        if plan is None:
+            if len(_PLANS) >= 32:
+                _PLANS.clear()
+            plan = _PLANS[key] = cls(*key)
+        return plan
+
+    def __init__(self, keys, R, itemsize, limits, cus):
+        groups = None
+        # strips much higher than the compute units ask for are not looked at
+        # unless the others do not do
+        rows = max(16, 4 * -(-sum(k[0][0] for k in keys) // cus))
+        for most in (rows, max(k[0][0] for k in keys)):
+            memo = {k: ShotStrips(k[0], k[1], R, itemsize, limits, k[2], most) for k in set(keys)}
+            groups = plan_groups([memo[k] for k in keys], cus)
+            if groups is not None:
+                break
+        self.ok = groups is not None
+        if not self.ok:
+            return
+        self.cost, groups = groups
+        cuts = [memo[k] for k in keys]
+        self.nzc = np.array([c.nzc for c in cuts])
+        strips, templates, row_strip = [], {}, []
+        self.group_begin, self.row_base = [0], []
+        n_rows = 0
+        for shots, cut in groups:
+            for si, parts in zip(shots, cut):
+                c = cuts[si]
+                self.row_base.append(n_rows)
+                n_rows += c.nx
+                for i, (x0, nr, xtype) in enumerate(parts):
+                    lay = c.layout(nr, xtype, len(parts) == 1)
+                    key = (lay, xtype, c.nzc, c.zfl, c.zfr)
+                    if key not in templates:
+                        templates[key] = (len(templates), thread_items(lay, xtype, c.nzc, c.zfl, c.zfr, R, limits))
+                    me = len(strips)
+                    up, down = i > 0, i + 1 < len(parts)
+                    d = [0] * STRIP_INTS
+                    d[0:4] = si, x0, nr, XTYPE if xtype else 0
+                    if up and xtype and parts[i - 1][2]:
+                        d[3] |= PXTOP
+                    if down and xtype and parts[i + 1][2]:
+                        d[3] |= PXBOT
+                    d[4:6] = (c.nzc, 0) if xtype else (c.zfl, c.zfr)
+                    d[6:8] = c.zfl, c.zfr
+                    d[19:24] = me - 1 if up else -1, me + 1 if down else -1, c.nzc, me, lay.exchange
+                    d[28] = templates[key][0]
+                    strips.append(d)
+                    row_strip.append(np.full(nr, me))
+            self.group_begin.append(len(strips))
+        self.strips = np.array(strips, dtype=np.int64)
+        self.row_strip = np.concatenate(row_strip)
+        self.row_base = np.array(self.row_base)
+        tables = [t for _, t in templates.values()]
+        self.items = np.stack([t[0] for t in tables])
+        # owners of the cells of all templates, (thread, step) a cell
+        self.owner = np.concatenate([t[1].reshape(-1, 2) for t in tables])
+        self.owner_base = np.cumsum([0] + [t[1].shape[0] * t[1].shape[1] for t in tables])
+
+
+class ResidentTables(object):
+    """Device tables of one batch for the resident loop (``build`` returns
+    None where the batch does not suit it)."""
+
+    _err = {}
+
+    @classmethod
+    def build(cls, batch, always=False):
+        import torch
+        if batch.dim != 2 or batch.adj_inj is None:
+            return None
+        limits = N.resident_limits()
+        item = batch.dtype.itemsize
+        most = cls._source_cells_per_row(batch.shots, 16 // item)
+        keys = tuple((tuple(int(n) for n in s.shape), tuple((l.size, r.size) for l, r in s.kpml), int(m))
+                     for s, m in zip(batch.shots, most))
+        cus = torch.cuda.get_device_properties(batch.dev).multi_processor_count
+        plan = Plan.of(keys, batch.R, item, limits, cus)
+        if not plan.ok:
+            return None
+        # few nodes in costly strips (thick PML, FP64 of order 8) step faster
+        # through the caches: 116 x 288 nodes in FP64 at cost 113 takes 11.1 us
+        # here and 8.6 there, 104 x 104 (4 shots, cost 53) 10.9 and 9.2; at
+        # cost 53, 448 x 175 in FP64 takes 11.8 and 12.0
+        nodes = sum(k[0][0] * k[0][1] for k in keys)
+        if not always and plan.cost > STEP_KERNEL_COST + nodes * item / STEP_KERNEL_BYTES:
+            return None
+        return cls(batch, plan, limits)
+
+    @staticmethod
+    def _source_cells_per_row(shots, V):
+        """Per shot, the most source cells in any of its rows, forward or
+        adjoint."""
+        most = np.zeros(len(shots), dtype=np.int64)
+        nx, nz = (max(s.shape[i] for s in shots) for i in range(2))
+        cells = -(-nz // V)
+        for way in range(2):
+            pos = [(s.src, s.adj)[way][0] for s in shots]
+            si = np.repeat(np.arange(len(shots)), [p.shape[0] for p in pos])
+            if si.size:
+                pos = np.concatenate(pos)
+                some = np.zeros(len(shots) * nx * cells, dtype=bool)
+                some[(si * nx + pos[:, 0]) * cells + pos[:, 1] // V] = True
+                most = np.maximum(most, some.reshape(len(shots), nx, cells).sum(axis=2, dtype=np.int32).max(axis=1))
+        return most
+
+    def __init__(self, batch, plan, limits):
+        import torch
+        dev, R, item = batch.dev, batch.R, batch.dtype.itemsize
+        V = 16 // item
+        hc = -(-R // V)
+        strips = plan.strips.copy()
+        n = len(strips)
+        nz = np.array([s.shape[1] for s in batch.shots])
+        # nodes numbered over the shots, thus in strip order
+        base = np.cumsum([0] + [s.shape[0] * s.shape[1] for s in batch.shots])
+
+        def place(node):
+            """(strip, row in it, z) of nodes."""
+            si = np.searchsorted(base, node, side="right") - 1
+            x, z = np.divmod(node - base[si], nz[si])
+            st = plan.row_strip[plan.row_base[si] + x]
+            return st, x - strips[st, 1], z
+
+        inj, fcells = [], np.zeros(n, dtype=np.int64)
+        for way, entries in enumerate(([s.src for s in batch.shots], [s.adj for s in batch.shots])):
+            si = np.repeat(np.arange(len(entries)), [e[0].shape[0] for e in entries])
+            pos, chan, w = (np.concatenate([e[i] for e in entries]) for i in range(3))
+            t = self._sources(plan, strips, place, base[si] + pos[:, 0] * nz[si] + pos[:, 1], chan, w, si, V, way)
+            fcells = np.maximum(fcells, t.pop("cells"))
+            inj.append(t)
+        strips[:, 24:28] = np.stack(lds_copies(strips, hc, R, fcells), axis=1)
+        strips[:, 14:19] = lds_offsets(strips[:, 24:28].T, strips[:, 2], item).T
+        # receiver nodes, in strip order
+        node = np.concatenate([b + idx for b, idx in zip(base, batch._rec_sorted)])
+        node, rec_node = _sorted_unique(node)
+        st, row, z = place(node)
+        rec_lds = (R + row) * (strips[st, 21] + hc) * 16 + hc * 16 + z * item
+        strips[:, 8] = np.searchsorted(st, np.arange(n))
+        strips[:, 9] = np.searchsorted(st, np.arange(n), side="right")
+        self.n_rec_nodes = node.size
+
+        # one upload, every table from a multiple of 16 bytes on
+        tables = [strips, plan.items, rec_lds, rec_node]
+        for t in inj:
+            tables += [t[k] for k in ("finfo", "lds", "nptr", "chan", "shot")]
+        at, size = [], 0
+        for t in tables:
+            at.append(size)
+            size += -(-t.size // 4) * 4
+        weights = [np.ascontiguousarray(t["w"], dtype=np.float64).view(np.int32) for t in inj]
+        w_at = [size, size + weights[0].size]
+        # (numpy: a tensor's fill wakes torch's threads, which then compete
+        # with numpy's for milliseconds)
+        flat = np.zeros(size + weights[0].size + weights[1].size + 4, dtype=np.int32)
+        for a, t in zip(at + w_at, tables + weights):
+            flat[a:a + t.size] = t.reshape(-1)
+        self._tables = torch.from_numpy(flat).to(dev)
+        ptr = self._tables.data_ptr()
+        self.n_inj = [int(t["lds"].size) for t in inj]
+        self.n_strips, self.cost = n, plan.cost
+        self.group_begin = np.asarray(plan.group_begin, dtype=np.int32)
+        self.group_lds = np.array([strips[a:b, 18].max() + 32 for a, b in zip(plan.group_begin[:-1], plan.group_begin[1:])],
+                                  dtype=np.int32)
+        cells = 2 * -(-int(strips[:, 21].max()) // 64) * 64 * R
+        stride = 2 * limits[4] * 4 + 4 * cells * 16
+        self.xchg = torch.zeros(n * stride // 4, dtype=torch.int32, device=dev)
+        self.epoch = ctypes.c_uint(0)
+        self._work = None
+        q = self.struct = N.Resident()
+        q.n_strips, q.n_groups = n, len(self.group_lds)
+        q.group_begin = self.group_begin.ctypes.data
+        q.group_lds = self.group_lds.ctypes.data
+        q.strips, q.items, q.rec_lds, q.rec_node = (ptr + 4 * a for a in at[:4])
+        for way in range(2):
+            (q.finfo[way], q.inj_lds[way], q.inj_nptr[way], q.inj_chan[way],
+             q.inj_shot[way]) = (ptr + 4 * a for a in at[4 + 5 * way:9 + 5 * way])
+            q.inj_w[way] = ptr + 4 * w_at[way]
+            q.n_inj[way] = self.n_inj[way]
+        q.n_rec_nodes = self.n_rec_nodes
+        q.xchg, q.xchg_stride, q.xchg_cells = self.xchg.data_ptr(), stride, cells
+        q.spin = SPIN
+        if dev not in ResidentTables._err:
+            ResidentTables._err[dev] = torch.zeros(16, dtype=torch.int32).pin_memory()
+        self.err = ResidentTables._err[dev]
+        q.err = self.err.data_ptr()
+        q.epoch = ctypes.addressof(self.epoch)
+
+    @staticmethod
+    def _sources(plan, strips, place, pos, chan, w, shot, V, way):
+        """Source tables in strip order: nodes, each with its entries in the
+        given order; for the strips with sources, per thread the first source
+        cell and the march steps that have one (a block of ``finfo``, which
+        the strip's number 29 + way names); source cells of every strip."""
+        n, threads = len(strips), plan.items.shape[1]
+        if pos.size and np.any(pos[1:] < pos[:-1]):
+            order = np.argsort(pos, kind="stable")
+            pos, chan, w, shot = (a[order] for a in (pos, chan, w, shot))
+        first = np.nonzero(np.concatenate([[True], pos[1:] != pos[:-1]]))[0] if pos.size else np.zeros(0, dtype=np.int64)
+        st, row, z = place(pos[first])
+        strips[:, 10 + 2 * way] = np.searchsorted(st, np.arange(n))
+        strips[:, 11 + 2 * way] = np.searchsorted(st, np.arange(n), side="right")
+        own = plan.owner[plan.owner_base[strips[st, 28]] + row * strips[st, 21] + z // V]
+        # a strip's cells in the order its threads march over them
+        key = (st * threads + own[:, 0]) * 64 + own[:, 1]
+        cells, inv = np.unique(key, return_inverse=True)
+        owner, step = cells // 64, cells % 64
+        begin = np.searchsorted(owner // threads, np.arange(n + 1))
+        lds = (inv.reshape(-1) - begin[st]) * V + z % V
+        some = np.nonzero(begin[1:] > begin[:-1])[0]
+        strips[:, 29 + way] = -1
+        strips[some, 29 + way] = np.arange(some.size)
+        finfo = np.zeros((max(1, some.size), threads, 2), dtype=np.int32)
+        if some.size:
+            heads = np.nonzero(np.concatenate([[True], owner[1:] != owner[:-1]]))[0]
+            k, t = np.divmod(owner[heads], threads)
+            finfo[strips[k, 29 + way], t, 0] = heads - begin[k]
+            finfo[strips[k, 29 + way], t, 1] = np.bitwise_or.reduceat(1 << step, heads)
+        return {"lds": lds, "nptr": np.append(first, pos.size), "chan": chan, "w": w, "shot": shot[first],
+                "finfo": finfo, "cells": np.diff(begin)}
+
+    def _workspace(self, batch):
+        """Source values and receiver nodes of a chunk of slots."""
+        import torch
+        if self._work is None or self._work[0] < min(batch.max_nt, self._chunk):
+            item = batch.dtype.itemsize
+            per_slot = (max(self.n_inj) + self.n_rec_nodes + 1) * item
+            self._chunk = max(32, CHUNK_BYTES // per_slot)
+            slots = min(batch.max_nt, self._chunk)
+            pre = torch.empty(slots * max(1, max(self.n_inj)), dtype=batch.tdtype, device=batch.dev)
+            rec = torch.empty(slots * max(1, self.n_rec_nodes), dtype=batch.tdtype, device=batch.dev)
+            self._work = (slots, pre, rec)
+            q = self.struct
+            q.pre, q.recbuf = pre.data_ptr(), rec.data_ptr()
+            q.pre_slots = q.rec_slots = slots
+
+    def check(self):
+        """Raise if an earlier run's wait for a neighbour ran into its bound."""
+        if int(self.err[0]):
+            self.err[0] = 0
+            raise N.NativeError("the resident time loop waited too long for a neighbouring strip; its results are "
+                                "not valid")
+
+    def run(self, batch, b, mode, j0, j1, direction, seg_base, record, stream):
+        self.check()
+        self._workspace(batch)
+        if self.epoch.value > 0xF0000000:
+            # the step tags wrap: start again from a cleared buffer
+            self.xchg.zero_()
+            self.epoch.value = 0
+        N.call("pysit_amd_resident_run", ctypes.byref(b), ctypes.byref(self.struct), mode, j0, j1, direction,
+               seg_base, 1 if record else 0, stream)

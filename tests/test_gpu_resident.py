@@ -1,0 +1,111 @@
+"""The 2D time loop with the wavefield held on the chip (GPU tests, through
+pysit_amd_resident_run): every result equals the one-launch-per-step loop bit
+for bit."""
+import numpy as np
+import pytest
+
+from tests.problems import Synthetic
+from tests.test_gpu_graph import _batch, _gradient, _same, _uneven
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(probs, dtype, **kw):
+    """The same batch on the step kernels and on the resident loop."""
+    return _batch(probs, dtype, 0, **kw), _batch(probs, dtype, None, resident=True, **kw)
+
+
+def _check(probs, dtype, res, segment=None, **kw):
+    steps, held = _pair(probs, dtype, **kw)
+    assert held.resident_tables() is not None and steps.resident_tables() is None
+    ref = _gradient(steps, res, segment=segment)
+    for rep in range(2):
+        out = _gradient(held, res, segment=segment)
+        assert _same(out[0], ref[0]), f"traces, pass {rep}"
+        assert _same(out[1], ref[1]), f"images, pass {rep}"
+    assert held.resident_tables().epoch.value > 0  # the runs above went through it
+    return steps, held
+
+
+def _residuals(probs, seed=9):
+    rng = np.random.default_rng(seed)
+    return [rng.standard_normal((p.nt, p.n_rec)) for p in probs]
+
+
+# (shape, PML widths): strips of every kind -- no room between the x sides, one
+# strip per side, a single middle strip, many strips; z rows of one cell more or
+# less than whole cells, rows wholly inside the PML, no PML on a side
+SHAPES = [((24, 30), ((4, 5), (6, 4))), ((61, 53), ((6, 7), (5, 8))), ((150, 65), ((10, 8), (7, 9))),
+          ((90, 260), ((0, 9), (0, 6))), ((333, 41), ((12, 12), (12, 12)))]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("order", [2, 4, 6, 8])
+@pytest.mark.parametrize("shape,pml", SHAPES)
+def test_resident_loop_equals_step_launches(gpu, dtype, order, shape, pml):
+    p = Synthetic(shape, pml, (0.01, 0.012), 83, order, seed=order, n_rec=9)
+    print("resident", shape, order, np.dtype(dtype).name, flush=True)
+    _check([p], dtype, _residuals([p]))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("segment", [None, 30])
+def test_resident_loop_uneven_shots_and_segments(gpu, dtype, segment):
+    probs = _uneven()
+    print("resident uneven", np.dtype(dtype).name, segment, flush=True)
+    _check(probs, dtype, _residuals(probs), segment=segment)
+
+
+@pytest.mark.parametrize("window", [7, 32])
+def test_resident_loop_windows_and_chunks(gpu, window, monkeypatch):
+    """FP32 windows that end inside launches and at their ends: the source and
+    receiver buffers hold 32 slots here, so a run takes many launches."""
+    from pysit_amd import resident
+    monkeypatch.setattr(resident, "CHUNK_BYTES", 1)
+    p = Synthetic((90, 110), ((10, 10), (10, 10)), (0.01, 0.01), 300, 8, seed=4)
+    for seg in (None, 50):
+        print("resident window", window, seg, flush=True)
+        _check([p], np.float32, _residuals([p], 7), segment=seg, ic_window=window)
+
+
+@pytest.mark.parametrize("kw", [{"imaging_period": 3}, {"adjoint": "exact"}])
+def test_resident_loop_imaging_period_and_exact_adjoint(gpu, kw):
+    p = Synthetic((70, 75), ((6, 7), (5, 8)), (0.01, 0.012), 90, 8, seed=2)
+    for dtype in (np.float64, np.float32):
+        print("resident", kw, np.dtype(dtype).name, flush=True)
+        _check([p], dtype, _residuals([p], 1), **kw)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_resident_loop_born_and_groups(gpu, dtype, monkeypatch):
+    """Born runs, and shots that run in several groups."""
+    from pysit_amd import resident
+    probs = [Synthetic((60, 75), ((6, 7), (5, 8)), (0.01, 0.012), 90, 8, seed=s, n_src=1 + s) for s in range(3)]
+    for p in probs[1:]:
+        p.model, p.Cpad, p.dt = probs[0].model, probs[0].Cpad, probs[0].dt
+    plan = resident.plan_groups
+    monkeypatch.setattr(resident, "plan_groups", lambda shots, cus: plan(shots, len(shots[0].cut(1e9))))
+    print("resident groups", np.dtype(dtype).name, flush=True)
+    steps, held = _check(probs, dtype, _residuals(probs))
+    assert len(held.resident_tables().group_lds) > 1
+    m1 = np.random.default_rng(4).standard_normal(probs[0].model.shape)
+    outs = []
+    for b in (steps, held):
+        b.forward(keep_dw=True, segment=probs[0].nt)
+        outs.append([t.cpu().numpy().copy() for t in b.born(m1)])
+    assert _same(outs[0], outs[1])
+
+
+def test_resident_wait_bound_is_an_error(gpu):
+    """A wait beyond its bound ends the launch and is reported: the host marks
+    the run as one that waited too long, without any kernel that does."""
+    from pysit_amd import _native as N
+    p = Synthetic((61, 53), ((6, 7), (5, 8)), (0.01, 0.012), 40, 4, seed=3)
+    steps, held = _pair([p], np.float64)
+    ref = _gradient(steps, _residuals([p]))
+    t = held.resident_tables()
+    t.err[0] = 1
+    with pytest.raises(N.NativeError, match="waited too long"):
+        held.forward(keep_dw=True)
+    out = _gradient(held, _residuals([p]))
+    assert _same(out[0], ref[0]) and _same(out[1], ref[1])

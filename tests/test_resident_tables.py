@@ -1,0 +1,87 @@
+"""The host tables of the resident 2D time loop (resident.py): every cell has
+one owner that marches over it, and what a thread reads and writes stays within
+its strip and its border rows."""
+import random
+
+import numpy as np
+import pytest
+
+from pysit_amd import resident
+
+# rows of a thread's column (plain, PML), threads, jobs of an exchange wave,
+# tags of a border: as the library reports them
+LIMITS = (9, 7, 512, 6, 64)
+
+
+def check_strip(plan, d, R):
+    nr, nzc, fl, fr = int(d[2]), int(d[21]), int(d[4]), int(d[5])
+    items = plan.items[d[28]]
+    a = plan.owner_base[d[28]]
+    owner = plan.owner[a:a + nr * nzc].reshape(nr, nzc, 2)
+    assert (owner >= 0).all()
+    cells, exchange = 0, 0
+    for w in range(LIMITS[2] // 64):
+        wave = items[64 * w:64 * w + 64].astype(np.int64)
+        kind = (wave[0, 1] // resident.KIND) & 3
+        assert ((wave[:, 1] // resident.KIND & 3) == kind).all()
+        if kind == 3:
+            exchange += wave[0, 0] < d[23]
+            continue
+        rows_most = LIMITS[0] if kind == 1 else LIMITS[1]
+        first = (wave[0, 2] >> 16) & 0xff
+        assert ((wave[:, 2] >> 16 & 0xff) == first).all()
+        for t, (base, flags, bits, where) in enumerate(wave):
+            col, alias = where & 0xffff, where >> 16
+            assert 0 <= alias < LIMITS[2] and items[alias, 3] & 0xffff == col
+            step = -1 if flags & resident.REV else 1
+            if not bits & 0xffff:  # nothing of its own: the same march as the thread it repeats
+                assert items[alias, 2] & 0xffff and (items[alias, :2] & 1).tolist() == [base & 1, flags & 1]
+                assert items[alias, 0] == base
+            own = [j for j in range(rows_most) if bits >> j & 1]
+            late = bits >> 24 & 1
+            assert not own or own == list(range(first + late, rows_most))
+            assert (fl <= col < nzc - fr) == (kind == 1)
+            for j in range(first, rows_most):
+                assert 0 <= base + step * j < nr
+            # the rows of the stencil around the march
+            for j in (first - R, rows_most - 1 + R):
+                assert -R <= base + step * j < nr + R
+            for j in own:
+                assert tuple(owner[base + step * j, col]) == (64 * w + t, j)
+                cells += 1
+            rows = [base + step * j for j in own]
+            if rows:
+                top, bot = flags & (2 | 32), flags & (4 | 64)
+                assert bool(top) == (min(rows) < R) and bool(bot) == (max(rows) + R >= nr)
+                # a march waits at its begin for the border it starts at
+                assert not (flags & (4 | 32) if step > 0 else flags & (2 | 64))
+    assert cells == nr * nzc and exchange == d[23] >= 1
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_tables_cover_the_grid_and_stay_in_bounds(seed):
+    rng = random.Random(seed)
+    held = 0
+    for _ in range(12):
+        shape = (rng.randint(12, 1200), rng.randint(10, 1500 if seed % 2 else 400))
+        pml = tuple(tuple(min(rng.choice([0, rng.randint(1, 25)]), n // 3) for _ in range(2)) for n in shape)
+        R, item = rng.randint(1, 4), rng.choice([4, 8])
+        keys = ((shape, pml, rng.randint(1, 3)),) * rng.choice([1, 2, 5, 20])
+        plan = resident.Plan(keys, R, item, LIMITS, 256)
+        if not plan.ok:
+            continue
+        held += 1
+        strips = plan.strips
+        assert np.diff(plan.group_begin).max() <= 256
+        for si in range(len(keys)):
+            mine = strips[strips[:, 0] == si]
+            assert mine[0, 1] == 0 and mine[-1, 1] + mine[-1, 2] == shape[0]
+            assert (mine[1:, 1] == mine[:-1, 1] + mine[:-1, 2]).all() and (len(mine) == 1 or (mine[:, 2] >= R).all())
+            assert (mine[:, 19] == np.append(-1, mine[:-1, 22])).all()
+            assert (mine[:, 20] == np.append(mine[1:, 22], -1)).all()
+        copies = np.stack(resident.lds_copies(strips, -(-R // (16 // item)), R, strips[:, 2] * keys[0][2]))
+        assert resident.lds_offsets(copies, strips[:, 2], item)[-1].max() + 32 <= resident.LDS_BYTES
+        _, one = np.unique(strips[:, 28], return_index=True)
+        for k in one:
+            check_strip(plan, strips[k], R)
+    assert held
