@@ -7,7 +7,7 @@
 // Shots are independent and a shot's fields are small, so here a launch keeps
 // them in registers and LDS for hundreds of steps: only the forward history
 // (dWaveOp, written or read once per step), the receivers' nodes and the rows
-// at strip borders move.  Now 17.5 and 23.0 us for the 16 shots, 3.3 us for
+// at strip borders move.  Now 18.1 and 20.3 us for the 16 shots, 3.2 us for
 // the small one; bound by the vector instructions of the PML rows (6 times a
 // plain row's), with few strips by the exchange of border rows.
 //
@@ -58,9 +58,12 @@ namespace pa {
 constexpr int kResThreads = 512;
 // rows of a thread's cell column: registers for du, C^2, the imaging sums and
 // the prefetched history (16 B per row each) plus the march's window fill the
-// 256 VGPRs that two waves per SIMD leave
+// 256 VGPRs that two waves per SIMD leave.  PML rows: with 7 the FP32 adjoint
+// spilled 18 registers, 23.7 us a step of 16 shots of 1041 x 341 nodes of
+// order 8; with 6 (2 spilled) 20.3, with 5 (none) 20.3 and the forward with
+// its store 18.7 instead of 19.4.
 constexpr int kPlainRows = 9;
-constexpr int kFullRows = 7;
+constexpr int kFullRows = 5;
 constexpr int kStripInts = 32;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -141,7 +144,6 @@ struct ResCtx {
     int gb, gstep;        // byte offset in a field of the shot of row j = 0, bytes per row
     int own, first;       // rows this thread owns (bit per j), first row of the wave
     bool late;            // the wave's first row is not this thread's
-    int alias;            // the thread whose cells a lane without rows repeats, else its own
     int drop;             // LDS byte offset of a cell nobody reads
     int rbase, dir, nr, col;
     int flags;            // item flags
@@ -544,7 +546,8 @@ __device__ __forceinline__ void strip_loop(const pysit_amd_batch &B, const ResPa
         Z.exact = B.dw_form == 1;
     }
     const int fblk = P.adjoint_tables ? d[30] : d[29];
-    const int2 fi = P.n_inj && fblk >= 0 ? P.finfo[(long long)fblk * kResThreads + c.alias] : make_int2(0, 0);
+    const int2 fi = P.n_inj && fblk >= 0 ? P.finfo[(long long)fblk * kResThreads +
+                                                             (P.items[d[28] * kResThreads + threadIdx.x].w >> 16)] : make_int2(0, 0);
     const int fp = d[16] + fi.x * 16;
     c.fany = 0;
     for (int j = 0; j < RM; ++j) c.fany |= __builtin_amdgcn_ballot_w64((fi.y >> j) & 1) ? 1 << j : 0;
@@ -861,7 +864,6 @@ __global__ __launch_bounds__(kResThreads) void k_resident2d(const pysit_amd_batc
     c.first = __builtin_amdgcn_readfirstlane((it.z >> 16) & 0xff);
     c.late = (it.z >> 24) & 1;
     c.col = it.w & 0xffff;
-    c.alias = it.w >> 16;
     c.dir = (it.y & I_REV) ? -1 : 1;
     c.nr = d[2];
     c.lwb = lwb;

@@ -10,7 +10,7 @@ from pysit_amd import resident
 
 # rows of a thread's column (plain, PML), threads, jobs of an exchange wave,
 # tags of a border: as the library reports them
-LIMITS = (9, 7, 512, 6, 64)
+LIMITS = (9, 5, 512, 6, 64)
 
 
 def check_strip(plan, d, R):
