@@ -456,6 +456,22 @@ __device__ __forceinline__ void store_rows(const C &c, Rsrc r, const Cell<T> (&a
     for (int j = 0; j < RM; ++j) cell_st<T>(r, (c.own >> j) & 1 ? c.gb + j * c.gstep : kOOB, a[j]);
 }
 
+// The flush of an FP32 window for a strip whose shot takes no step in the
+// launch: a window that another run left open (the step kernels, in a segment
+// too short for this loop) ends here if one of the launch's slots ends it.
+// ic += sums, sums = 0 over the strip's rows, as k_ic_flush does.
+__device__ __forceinline__ void flush_idle(const pysit_amd_batch &B, const pysit_amd_shot &S, const int (&d)[kStripInts],
+                                           int slot_begin, int slot_end, int window)
+{
+    if ((slot_begin + window - 1) / window * window >= slot_end) return;
+    float *sum = B.ic32 + S.off + (long long)d[1] * S.zs;
+    double *ic = B.ic + S.off + (long long)d[1] * S.zs;
+    for (int i = threadIdx.x; i < d[2] * S.zs; i += kResThreads) {
+        ic[i] += (double)sum[i];
+        sum[i] = 0.0f;
+    }
+}
+
 // the FP32 window's flush: ic += sums, sums = 0
 template <int RM, typename C>
 __device__ __forceinline__ void flush_rows(const C &c, Rsrc ric, Cell<float> (&ic)[RM])
@@ -831,7 +847,10 @@ __global__ __launch_bounds__(kResThreads) void k_resident2d(const pysit_amd_batc
     const int first_slot = P.direction > 0 ? lo : end - 1;
     // receivers of a shot that starts inside the launch: its earlier slots
     // hold no values and are not read
-    if (n <= 0) return;
+    if (n <= 0) {
+        if constexpr (MODE == 4) flush_idle(B, S, d, P.slot_begin, end, P.window);
+        return;
+    }
 
     for (int i = tid; i < d[18] / 16 + 2; i += kResThreads)
         *reinterpret_cast<u32x4 *>(smem + 16 * i) = u32x4{0, 0, 0, 0};

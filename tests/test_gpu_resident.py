@@ -109,3 +109,24 @@ def test_resident_wait_bound_is_an_error(gpu):
         held.forward(keep_dw=True)
     out = _gradient(held, _residuals([p]))
     assert _same(out[0], ref[0]) and _same(out[1], ref[1])
+
+
+@pytest.mark.parametrize("window", [7, 64])
+def test_fp32_window_of_a_shot_that_starts_in_a_short_segment(gpu, window):
+    """A shot whose step 0 lies in a segment too short for the resident loop:
+    the step kernels leave its FP32 window open, and the window's end lies in
+    a segment where the shot takes no step."""
+    base = Synthetic((60, 50), ((6, 6), (5, 5)), (0.01, 0.01), 97, 8, seed=3, src_center=(30, 8))
+    probs = [base] + [Synthetic((60, 50), ((6, 6), (5, 5)), (0.01, 0.01), nt, 8, seed=40 + nt, model=base.model,
+                                dt=base.dt, src_center=(30, 8)) for nt in (5, 7, 36, 68)]
+    res = _residuals(probs, 3)
+    steps, held = _pair(probs, np.float32, ic_window=window)
+    ref = _gradient(steps, res)
+    assert all(np.abs(i).max() > 0 for i in ref[1])
+    short = []  # lengths of the runs that the step kernels took
+    run = held._resident_for
+    held._resident_for = lambda b, mode, n: run(b, mode, n) or short.append((mode, n))
+    # slots 90 to 96 are a segment of 7: the shots of 5 and 7 steps live in it
+    out = _gradient(held, res, segment=30)
+    assert (2, 7) in short and held.resident_tables().epoch.value > 0
+    assert _same(out[0], ref[0]) and _same(out[1], ref[1])
