@@ -198,6 +198,18 @@ template <typename T, int R> __device__ __forceinline__ void wait_borders(const 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Whether step i of the launch is a strip's last because a poll ran into its
+// bound in it: `bad` holds 1 + that step.  A wave may read the word late, when
+// an exchange wave is already in the next step and its poll expires there; by
+// the number all waves leave after the same step, whose border rows have been
+// counted.  One that left a step early would leave the others waiting for its
+// count.
+__device__ __forceinline__ bool last_step(const int *bad, int i)
+{
+    const int at = lds_word(bad);
+    return at != 0 && at <= i + 1;
+}
+
 constexpr bool res_back(int mode) { return mode == 2 || mode == 4; }
 constexpr bool res_reads(int mode) { return mode >= 2; }
 
@@ -619,7 +631,7 @@ __device__ __forceinline__ void strip_loop(const pysit_amd_batch &B, const ResPa
         c.pzw2 = -c.pzw2;
         f_at = fp + ((i + 1) & 1) * d[27];
         lds_sync();
-        bad = lds_word(reinterpret_cast<const int *>(c.smem + c.flag + 8)) != 0;
+        bad = last_step(reinterpret_cast<const int *>(c.smem + c.flag + 8), i);
         if (bad) break;
     }
     // state back to memory; after a poll that ran into its bound, NaN
@@ -682,7 +694,7 @@ __device__ __forceinline__ void exchange_loop(const ResParams<T> &P, const int (
         lds_sync();
         for (int i = 0; i < n; ++i) {
             lds_sync();
-            if (lds_word(bad)) break;
+            if (last_step(bad, i)) break;
         }
         return;
     }
@@ -774,7 +786,7 @@ __device__ __forceinline__ void exchange_loop(const ResParams<T> &P, const int (
             // the neighbour may be a step ahead: its other buffer holds this one
             while (tagged && (int)(__hip_atomic_load(get, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - tag) < 0)
                 if (++spins > P.spin) {
-                    __hip_atomic_store(bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_store(bad, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     break;
                 }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -819,7 +831,7 @@ __device__ __forceinline__ void exchange_loop(const ResParams<T> &P, const int (
                 *reinterpret_cast<T *>(smem + d[16] + P.inj_lds[q] * SZ + fn) = pn[q - inj0];
         }
         lds_sync();
-        if (lds_word(bad)) {
+        if (last_step(bad, i)) {
             if (lane == 0) __hip_atomic_store(P.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             break;
         }

@@ -130,3 +130,28 @@ def test_fp32_window_of_a_shot_that_starts_in_a_short_segment(gpu, window):
     out = _gradient(held, res, segment=30)
     assert (2, 7) in short and held.resident_tables().epoch.value > 0
     assert _same(out[0], ref[0]) and _same(out[1], ref[1])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_resident_expired_wait_ends_the_launch(gpu, dtype):
+    """Waits with a bound of one poll expire in many strips at different
+    steps: every launch ends, the run is reported, and the runs after it are
+    whole again."""
+    import torch
+    from pysit_amd import _native as N
+    from pysit_amd import resident
+    p = Synthetic((333, 141), ((12, 12), (12, 12)), (0.01, 0.01), 200, 8, seed=5)
+    steps, held = _pair([p], dtype)
+    ref = _gradient(steps, _residuals([p]))
+    t = held.resident_tables()
+    assert t.n_strips > 8
+    t.struct.spin = 1
+    print("resident expired wait", np.dtype(dtype).name, flush=True)
+    held.forward(keep_dw=True)
+    torch.cuda.synchronize()
+    assert int(t.err[0]) == 1
+    t.struct.spin = resident.SPIN
+    with pytest.raises(N.NativeError, match="waited too long"):
+        held.forward(keep_dw=True)
+    out = _gradient(held, _residuals([p]))
+    assert _same(out[0], ref[0]) and _same(out[1], ref[1])
