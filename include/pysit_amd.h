@@ -359,9 +359,11 @@ int pysit_amd_plan_destroy(pysit_amd_plan *plan);
 /* Shots run in groups of at most one strip per compute unit.  The tables    */
 /* are built on the host (pysit_amd/resident.py).  A launch is cooperative:  */
 /* not for streams under capture.  The waits for a neighbour are bounded;    */
-/* one that reaches the bound (`spin` polls of about 1 us) ends the launch,  */
-/* leaves NaN in the state and writes 1 to *err, which the caller checks     */
-/* once the stream has been waited for.                                      */
+/* one that reaches the bound (`spin` polls of about 1 us) ends its strip    */
+/* and writes 1 to *err, which the caller checks once the stream has been    */
+/* waited for, and to *stop: later launches take no step and leave NaN in    */
+/* the state.  Traces, histories and sums of such runs are not valid until   */
+/* pysit_amd_resident_seal turns traces and image into NaN.                  */
 /* ------------------------------------------------------------------------ */
 typedef struct {
     int n_strips, n_groups;
@@ -391,6 +393,7 @@ typedef struct {
     int xchg_cells;          /* cells of 16 bytes, at most, of one border       */
     int spin;
     int *err;                /* host memory the device can write                */
+    int *stop;               /* device word, 0 before the first run             */
     unsigned *epoch;         /* HOST: next step tag, 0 before the first run     */
 } pysit_amd_resident;
 
@@ -403,6 +406,10 @@ int pysit_amd_resident_limits(int *limits);
  * the receivers (modes 0, 1 and 3). */
 int pysit_amd_resident_run(const pysit_amd_batch *b, const pysit_amd_resident *r, int mode, int slot_begin,
                            int slot_end, int direction, int seg_base, int record, void *stream);
+
+/* Queued behind the runs of a forward or an adjoint: if a wait expired, NaN
+ * into b's image (b->ic, if given) and, with b->n_rec, into every trace. */
+int pysit_amd_resident_seal(const pysit_amd_batch *b, const pysit_amd_resident *r, void *stream);
 
 /* Sum of squares over time slots of a slot-major store (the dWaveOp store):
  * out[i] += sum over s = slot_begin, slot_begin + slot_step, ... < slot_end of

@@ -65,7 +65,7 @@ class Resident(ctypes.Structure):
         ("rec_lds", _vp), ("n_rec_nodes", _i), ("rec_node", _vp),
         ("pre", _vp), ("pre_slots", _i), ("recbuf", _vp), ("rec_slots", _i),
         ("xchg", _vp), ("xchg_stride", _ll), ("xchg_cells", _i), ("spin", _i),
-        ("err", _vp), ("epoch", _vp),
+        ("err", _vp), ("stop", _vp), ("epoch", _vp),
     ]
 
 
@@ -91,6 +91,7 @@ SIGNATURES = {
     "pysit_amd_batch_run_persistent": [ctypes.POINTER(Batch), _i, _i, _i, _i, _i, _vp, _vp, _vp],
     "pysit_amd_resident_limits": [_vp],
     "pysit_amd_resident_run": [ctypes.POINTER(Batch), ctypes.POINTER(Resident), _i, _i, _i, _i, _i, _i, _vp],
+    "pysit_amd_resident_seal": [ctypes.POINTER(Batch), ctypes.POINTER(Resident), _vp],
     "pysit_amd_fold": [_i] * 10 + [_vp, _d, _vp, _i, _i, _i, _vp],
     "pysit_amd_slot_square_sum": [_vp, _i, _ll, _i, _i, _i, _ll, _vp, _vp],
     "pysit_amd_plan_create": [_i, _i, ctypes.POINTER(_vp)],

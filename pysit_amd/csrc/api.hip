@@ -24,6 +24,7 @@ int run2d_persistent(const pysit_amd_batch &, int, int, int, int, int, const int
 
 template <typename T>
 int run2d_resident(const pysit_amd_batch &, const pysit_amd_resident &, int, int, int, int, int, int, hipStream_t);
+int resident_seal(const pysit_amd_batch &, const int *, hipStream_t);
 void resident_rows(int *plain, int *full, int *threads, int *ops, int *tags);
 
 int ic_flush(const pysit_amd_batch &B, hipStream_t st);
@@ -525,13 +526,21 @@ int pysit_amd_resident_run(const pysit_amd_batch *b, const pysit_amd_resident *r
     PA_CHECK(!B.fstore && !B.dw_out && !B.vol_dw, "the resident loop stores no field and has no second-order terms");
     PA_CHECK(mode == 2 ? direction == -1 : direction == 1, "the resident loop runs forward, its adjoint backward");
     PA_CHECK(r->n_groups >= 1 && r->group_begin && r->group_lds && r->strips && r->items && r->finfo[0] &&
-                 r->xchg && r->err && r->epoch && r->spin >= 1,
+                 r->xchg && r->err && r->stop && r->epoch && r->spin >= 1,
              "resident tables missing");
     if (slot_end <= slot_begin) return PYSIT_AMD_OK;
     return B.dtype ? run2d_resident<double>(B, *r, mode, slot_begin, slot_end, direction, seg_base, record,
                                             (hipStream_t)stream)
                    : run2d_resident<float>(B, *r, mode, slot_begin, slot_end, direction, seg_base, record,
                                            (hipStream_t)stream);
+}
+
+int pysit_amd_resident_seal(const pysit_amd_batch *b, const pysit_amd_resident *r, void *stream)
+{
+    clear_error();
+    PA_CHECK(b && r && r->stop, "null argument");
+    PA_CHECK(b->total_n >= 0 && b->n_shots >= 0 && (!b->n_rec || b->shots), "bad batch");
+    return resident_seal(*b, r->stop, (hipStream_t)stream);
 }
 
 int pysit_amd_slot_square_sum(const void *store, int dtype, long long slot_stride, int slot_begin, int slot_end,

@@ -41,8 +41,12 @@
 // instead of 2.4 for 341 FP32 nodes of order 8.
 //
 // All strips of a launch must run at the same time (a cooperative launch of
-// at most one workgroup per CU); every poll is bounded, a poll that reaches
-// the bound ends every workgroup, sets `err` and leaves NaN in the state.
+// at most one workgroup per CU).  Every poll is bounded.  One that reaches the
+// bound ends its strip, whose neighbours' polls then expire in turn, and sets
+// `err` and `stop`; strips of other shots run on.  Launches that find `stop`
+// set take no step.  The stopped strips leave NaN in the state, and
+// resident_seal, queued behind the runs, turns the traces and the image of the
+// whole batch into NaN.
 //
 // The arithmetic is that of cda2d.hip's batch steps, operation by operation,
 // so results equal the step loop's bit for bit.
@@ -90,7 +94,8 @@ struct ResParams {
     char *xchg;
     long long xstride;    // bytes per strip
     int xcells;           // cells of one border and time level
-    int *err;
+    int *err;             // host word and, for the launches behind this one, device word of an expired wait
+    int *stop;
     unsigned epoch;
     int strip0, slot_begin, n_steps, direction, seg_base;
     int n_inj, n_rec, adjoint_tables, record, window, spin;
@@ -601,8 +606,8 @@ __device__ __forceinline__ void strip_loop(const pysit_amd_batch &B, const ResPa
     lds_sync();
 
     const int jobs_top = border_jobs(d, 0), jobs_bot = border_jobs(d, 1);
-    bool bad = false;
-    for (int i = 0; i < n; ++i) {
+    bool bad = lds_word(reinterpret_cast<const int *>(c.smem + c.flag + 12)) != 0;
+    for (int i = 0; i < n && !bad; ++i) {
         const int slot = first_slot + i * P.direction, k = slot - kshift;
         const bool more = i + 1 < n;
         const bool img = res_imaged(B, k);
@@ -632,7 +637,6 @@ __device__ __forceinline__ void strip_loop(const pysit_amd_batch &B, const ResPa
         f_at = fp + ((i + 1) & 1) * d[27];
         lds_sync();
         bad = last_step(reinterpret_cast<const int *>(c.smem + c.flag + 8), i);
-        if (bad) break;
     }
     // state back to memory; after a poll that ran into its bound, NaN
     const Rsrc wu = make_rsrc((T *)B.u[fin] + S.off, nb);
@@ -692,6 +696,7 @@ __device__ __forceinline__ void exchange_loop(const ResParams<T> &P, const int (
     int *bad = f + 2;
     if (me >= d[23]) {  // an idle wave keeps the others company at the barriers
         lds_sync();
+        if (lds_word(bad + 1)) return;
         for (int i = 0; i < n; ++i) {
             lds_sync();
             if (last_step(bad, i)) break;
@@ -745,6 +750,7 @@ __device__ __forceinline__ void exchange_loop(const ResParams<T> &P, const int (
         *reinterpret_cast<T *>(smem + d[16] + P.inj_lds[i] * SZ) =
             P.pre[(long long)(first_slot - P.slot_begin) * P.n_inj + i];
     lds_sync();
+    if (lds_word(bad + 1)) return;
     for (int i = 0; i < n; ++i) {
         const int slot = first_slot + i * P.direction;
         const bool more = i + 1 < n;
@@ -832,7 +838,10 @@ __device__ __forceinline__ void exchange_loop(const ResParams<T> &P, const int (
         }
         lds_sync();
         if (last_step(bad, i)) {
-            if (lane == 0) __hip_atomic_store(P.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (lane == 0) {
+                __hip_atomic_store(P.stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(P.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
             break;
         }
     }
@@ -867,6 +876,10 @@ __global__ __launch_bounds__(kResThreads) void k_resident2d(const pysit_amd_batc
     for (int i = tid; i < d[18] / 16 + 2; i += kResThreads)
         *reinterpret_cast<u32x4 *>(smem + 16 * i) = u32x4{0, 0, 0, 0};
     lds_sync();
+    // one read for all waves, which look at it after their first barrier
+    if (tid == 0)
+        *reinterpret_cast<int *>(smem + d[18] + 12) =
+            __hip_atomic_load(P.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     {
         // x profiles of the strip's rows
         T *sg = reinterpret_cast<T *>(smem + d[17]);
@@ -959,7 +972,29 @@ __global__ __launch_bounds__(256) void k_rec_sum(const pysit_amd_batch B, const 
     }
 }
 
+// NaN into the traces and the image of a batch whose wait expired.  Queued
+// behind every forward and every adjoint: 256 workgroups that read one word.
+__global__ __launch_bounds__(256) void k_res_seal(const pysit_amd_batch B, const int *stop)
+{
+    if (!*stop) return;
+    const long long at = (long long)blockIdx.x * 256 + threadIdx.x, step = (long long)gridDim.x * 256;
+    if (B.ic)
+        for (long long i = at; i < B.total_n; i += step) B.ic[i] = __builtin_nan("");
+    if (!B.n_rec) return;
+    for (int s = 0; s < B.n_shots; ++s) {
+        const pysit_amd_shot &S = B.shots[s];
+        for (long long i = at; i < (long long)S.nt * S.nrec; i += step) S.trace[i] = __builtin_nan("");
+    }
+}
+
 // ---- host ---------------------------------------------------------------------
+int resident_seal(const pysit_amd_batch &B, const int *stop, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_res_seal, dim3(256), dim3(256), 0, st, B, stop);
+    PA_HIP(hipGetLastError());
+    return PYSIT_AMD_OK;
+}
+
 int inj_precompute(const pysit_amd_batch &B, int slot_begin, int slot_end, int seg_base, hipStream_t st);
 
 template <typename T, int R, int MODE>
@@ -1032,6 +1067,7 @@ int run2d_resident(const pysit_amd_batch &B, const pysit_amd_resident &Q, int mo
     P.xstride = Q.xchg_stride;
     P.xcells = Q.xchg_cells;
     P.err = Q.err;
+    P.stop = Q.stop;
     P.direction = direction;
     P.seg_base = seg_base;
     P.n_inj = mode == 3 ? 0 : Q.n_inj[adj];

@@ -853,6 +853,30 @@ class DeviceBatch:
             return None
         return tables
 
+    def check(self):
+        """Raise if a wait of the resident loop expired in a run whose results
+        the host has waited for: they are NaN.  The batch goes on with the
+        step kernels, and its histories of that run are dropped.  The host
+        calls of TemporalModeling check the results they return; a program
+        that takes device tensors checks once it has waited for them, or at
+        the batch's next run."""
+        if self._resident and self._resident.expired():
+            self._resident = False
+            self.generation += 1
+            self.have_dw = False
+            self.ckpts = []
+            self._dw_seg = None
+            self.dw1 = None
+            self.dw_adj = None
+            raise N.NativeError("the resident time loop waited too long for a neighbouring strip; its results are "
+                                "not valid (run again: the batch now steps launch by launch)")
+
+    def _seal(self, b):
+        """Behind the runs of a forward or an adjoint: no result of a run
+        whose wait expired looks like one."""
+        if self._resident and self._resident.epoch.value:
+            self._resident.seal(b, _stream())
+
     def _run(self, b, mode, j0, j1, direction, seg_base, record=True):
         at = np.ascontiguousarray(self.active_tiles)
         ar = np.ascontiguousarray(self.active_recs if record else np.zeros_like(self.active_recs))
@@ -976,6 +1000,7 @@ class DeviceBatch:
         at segment boundaries.  ``store_field`` also keeps u_k of every step
         (``field_store``).  Returns the per-shot traces (device FP64, in the
         caller's shot order)."""
+        self.check()
         self.generation += 1
         for t in self.traces:
             t.zero_()
@@ -998,7 +1023,9 @@ class DeviceBatch:
             # forward pass only records the traces
             if store_field:
                 raise ValueError("storing the wavefield needs the whole dWaveOp history in memory")
-            self._run(self._batch(self.fstate, False), 0, 0, self.max_nt, 1, 0)
+            b = self._batch(self.fstate, False)
+            self._run(b, 0, 0, self.max_nt, 1, 0)
+            self._seal(b)
             self.have_dw = True
             return self.traces_in_caller_order()
         if segment:
@@ -1037,6 +1064,7 @@ class DeviceBatch:
             b = self._batch(self.fstate, False)
             b.fstore = self.field_store.data_ptr() if store_field else None
             self._run(b, 0, 0, self.max_nt, 1, 0)
+        self._seal(b)
         self.have_dw = keep_dw
         return self.traces_in_caller_order()
 
@@ -1123,6 +1151,7 @@ class DeviceBatch:
         every step is kept in ``self.dw1`` (linear_forward_model's 'dWaveOp1'),
         with ``store_field`` u1 of every step in ``field_store``.  Returns
         per-shot traces (caller order)."""
+        self.check()
         if not getattr(self, "have_dw", False) or self.ckpts or self.imaging_period != 1:
             raise RuntimeError("born needs forward(keep_dw=True) with every step stored (imaging_period 1)")
         m1 = torch.as_tensor(np.ascontiguousarray(m1, dtype=self.dtype)).to(self.dev)
@@ -1145,6 +1174,7 @@ class DeviceBatch:
         self.field_store = self._field_store() if store_field else None
         b.fstore = self.field_store.data_ptr() if store_field else None
         self._run(b, 3, 0, self.max_nt, 1, 0)
+        self._seal(b)
         return self.traces_in_caller_order()
 
     def traces_in_caller_order(self):
@@ -1170,6 +1200,7 @@ class DeviceBatch:
         every step in ``self.dw_adj``; ``volume`` = (vol_m, history) adds the
         source vol_m * history_k (vol_m: a flat batch array, see
         padded_operand; history: a (max_nt, total_n) store)."""
+        self.check()
         second = image_store != "dw" or store_adjoint_dw or volume is not None
         binomial = image and self.snaps is not None
         if second and (self.imaging_period != 1 or (image and (self.ckpts or binomial))):
@@ -1265,6 +1296,10 @@ class DeviceBatch:
             for si in range(len(self.ckpts) - 1, -1, -1):
                 j0 = si * K
                 self._reverse(j0, min(self.max_nt, j0 + K), self.ckpts[si], 1, levels, work, fb, wb, qb)
+        self._seal(qb)
+        if self.dw_sq is not None:
+            qb.ic = self.dw_sq.data_ptr()
+            self._seal(qb)
         return self.ic
 
     def _treeverse(self, a, b, snaps, ckpt, work, fb, wb, qb):

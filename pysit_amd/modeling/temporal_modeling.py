@@ -25,6 +25,7 @@ Batched extensions run many shots in one launch per time step:
 """
 import numpy as np
 
+from .._native import NativeError
 from ..core.receivers import adjoint_entries, sampling_entries
 from ..device import DeviceBatch, ShotGeometry
 
@@ -46,6 +47,7 @@ class DWaveOpHandle(object):
 
     def __array__(self, dtype=None, copy=None):
         a = self.batch.shot_dw(self.shot, self.k, self.store).reshape(-1, 1).double().cpu().numpy()
+        self.batch.check()
         return a if dtype is None else a.astype(dtype)
 
 
@@ -89,6 +91,7 @@ class TemporalModeling(object):
         if adjoint not in ("pysit", "exact"):
             raise ValueError("adjoint must be 'pysit' or 'exact'")
         self.adjoint = adjoint
+        self._step_kernels = False  # a wait of the resident loop expired: later batches do without it
 
     # ---------------------------------------------------------------- plumbing
     def geometry(self, shot):
@@ -154,6 +157,8 @@ class TemporalModeling(object):
         s = self.solver
         kw = dict(dtype=s.dtype, imaging_period=imaging_period, memory_budget=self.memory_budget,
                   ic_window=self.ic_window, adjoint=self.adjoint)
+        if self._step_kernels:
+            kw["resident"] = False
         if self.autotune and not self.tile_x:
             if s.mesh.dim == 2:
                 b = DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
@@ -164,6 +169,16 @@ class TemporalModeling(object):
             return tuned_batch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
         return DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, tile_x=self.tile_x,
                            **kw)
+
+    def _host(self, batch, t):
+        """Result tensor ``t`` of ``batch`` on the host, checked."""
+        a = t.cpu().numpy()
+        try:
+            batch.check()
+        except NativeError:
+            self._step_kernels = True
+            raise
+        return a
 
     def _unpad_field(self, padded):
         mesh = self.solver.mesh
@@ -180,7 +195,7 @@ class TemporalModeling(object):
         else:
             for i in shots_idx:
                 batch.fold(i, mesh.pad_widths(), out, scale=scale, accumulate=True)
-        return s.model_parameters.without_padding().perturbation(data=out.cpu().numpy().reshape(-1, 1))
+        return s.model_parameters.without_padding().perturbation(data=self._host(batch, out).reshape(-1, 1))
 
     # ----------------------------------------------------------------- forward
     def forward_model(self, shot, m0, imaging_period=1, return_parameters=[]):
@@ -197,7 +212,7 @@ class TemporalModeling(object):
         if keep:
             retval["dWaveOp"] = _handles(b, 0, solver.nsteps, imaging_period)
         if "simdata" in return_parameters:
-            retval["simdata"] = traces[0].cpu().numpy()
+            retval["simdata"] = self._host(b, traces[0])
         return retval
 
     def forward_model_batch(self, shots, m0, imaging_period=1, keep_dw=False):
@@ -208,7 +223,7 @@ class TemporalModeling(object):
         b = self.batch(shots, imaging_period, reuse=True)
         traces = b.forward(keep_dw=keep_dw)
         self.last_batch = b if keep_dw else None
-        return [t.cpu().numpy() for t in traces]
+        return [self._host(b, t) for t in traces]
 
     # ----------------------------------------------------------------- adjoint
     def _batch_for(self, shot, dWaveOp, imaging_period):
@@ -317,7 +332,7 @@ class TemporalModeling(object):
         if device:
             ops = [operands_fn(i, t) for i, t in enumerate(traces)]
         else:
-            ops = [np.asarray(operands_fn(i, t.cpu().numpy()), dtype=np.float64) for i, t in enumerate(traces)]
+            ops = [np.asarray(operands_fn(i, self._host(b, t)), dtype=np.float64) for i, t in enumerate(traces)]
         b.migrate(ops, dw_squares=dw_squares)
         g = self._fold_images(b, -solver.dt * imaging_period)
         self.last_batch = b
@@ -345,7 +360,7 @@ class TemporalModeling(object):
                                     for k in range(solver.nsteps)]
             b.field_store = None
         if "simdata" in return_parameters:
-            retval["simdata"] = traces[si].cpu().numpy()
+            retval["simdata"] = self._host(b, traces[si])
         if "dWaveOp0" in return_parameters:
             retval["dWaveOp0"] = _handles(b, si, solver.nsteps, 1)
         if keep1:

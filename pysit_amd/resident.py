@@ -10,7 +10,10 @@ that do not fit the GPU together run one group after the other.
 Everything here is numpy on the host; :class:`ResidentTables` uploads the
 result once per batch geometry.
 """
+import collections
 import ctypes
+import threading
+import weakref
 
 import numpy as np
 
@@ -39,7 +42,36 @@ STEP_KERNEL_COST = 35.0
 STEP_KERNEL_BYTES = 30000.0
 # device memory for the source values and receiver nodes of a chunk of slots
 CHUNK_BYTES = 256 << 20
-SPIN = 1 << 20
+# polls of about 1 us (16 s) before a wait for a neighbour gives up: a strip
+# may start late where another stream's kernels hold compute units
+SPIN = 1 << 24
+
+
+class _Words(object):
+    """Pinned host words that a device can write, one per user: the word of
+    an expired wait belongs to one batch.  A freed word is the last to be
+    given out again: a launch of a batch that is gone may still write it."""
+
+    BLOCK = 1024
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._free = collections.deque()
+
+    def take(self, owner):
+        """A word (a view of one int32) that is ``owner``'s while it lives."""
+        import torch
+        with self._lock:
+            if not self._free:
+                block = torch.zeros(self.BLOCK, dtype=torch.int32).pin_memory()
+                self._free.extend(block[i:i + 1] for i in range(self.BLOCK))
+            word = self._free.popleft()
+        word[0] = 0
+        weakref.finalize(owner, self._free.append, word)
+        return word
+
+
+_WORDS = _Words()
 
 
 def z_columns(nz, nzl, nzr, R, V):
@@ -459,8 +491,6 @@ class ResidentTables(object):
     """Device tables of one batch for the resident loop (``build`` returns
     None where the batch does not suit it)."""
 
-    _err = {}
-
     @classmethod
     def build(cls, batch, always=False):
         import torch
@@ -577,10 +607,10 @@ class ResidentTables(object):
         q.n_rec_nodes = self.n_rec_nodes
         q.xchg, q.xchg_stride, q.xchg_cells = self.xchg.data_ptr(), stride, cells
         q.spin = SPIN
-        if dev not in ResidentTables._err:
-            ResidentTables._err[dev] = torch.zeros(16, dtype=torch.int32).pin_memory()
-        self.err = ResidentTables._err[dev]
+        self.err = _WORDS.take(self)
         q.err = self.err.data_ptr()
+        self._stop = torch.zeros(1, dtype=torch.int32, device=dev)
+        q.stop = self._stop.data_ptr()
         q.epoch = ctypes.addressof(self.epoch)
 
     @staticmethod
@@ -631,15 +661,17 @@ class ResidentTables(object):
             q.pre, q.recbuf = pre.data_ptr(), rec.data_ptr()
             q.pre_slots = q.rec_slots = slots
 
-    def check(self):
-        """Raise if an earlier run's wait for a neighbour ran into its bound."""
-        if int(self.err[0]):
-            self.err[0] = 0
-            raise N.NativeError("the resident time loop waited too long for a neighbouring strip; its results are "
-                                "not valid")
+    def expired(self):
+        """Whether a wait for a neighbour ran into its bound in a run that the
+        host knows of: all those before the last time it waited for them."""
+        return int(self.err[0]) != 0
+
+    def seal(self, b, stream):
+        """Behind the runs of a forward or an adjoint: NaN into the batch
+        descriptor's traces and image if a wait expired in any of them."""
+        N.call("pysit_amd_resident_seal", ctypes.byref(b), ctypes.byref(self.struct), stream)
 
     def run(self, batch, b, mode, j0, j1, direction, seg_base, record, stream):
-        self.check()
         self._workspace(batch)
         if self.epoch.value > 0xF0000000:
             # the step tags wrap: start again from a cleared buffer

@@ -155,3 +155,59 @@ def test_resident_expired_wait_ends_the_launch(gpu, dtype):
         held.forward(keep_dw=True)
     out = _gradient(held, _residuals([p]))
     assert _same(out[0], ref[0]) and _same(out[1], ref[1])
+
+
+def _one_poll(held):
+    """Waits of this batch give up after one poll."""
+    held.resident_tables().struct.spin = 1
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_results_of_an_expired_wait_are_nan(gpu, dtype):
+    """No trace and no image of a run whose wait expired holds a number, also
+    where the host has not seen it yet, and another batch's runs are not
+    touched."""
+    import torch
+    from pysit_amd import _native as N
+    p = Synthetic((333, 141), ((12, 12), (12, 12)), (0.01, 0.01), 200, 8, seed=5)
+    res = _residuals([p])
+    steps, held = _pair([p], dtype)
+    other = _batch([p], dtype, None, resident=True)
+    ref = _gradient(steps, res)
+    _one_poll(held)
+    print("resident expired results", np.dtype(dtype).name, flush=True)
+    tr = held.forward(keep_dw=True)[0].cpu()
+    assert torch.isnan(tr).all()
+    held.resident_tables().err[0] = 0  # as if the host had not waited yet
+    held.resident_tables().struct.spin = 1 << 20
+    ic = held.migrate(res)
+    assert torch.isnan(ic).all()
+    tr = held.forward(keep_dw=True)[0].cpu()
+    assert torch.isnan(tr).all()
+    out = _gradient(other, res)
+    assert _same(out[0], ref[0]) and _same(out[1], ref[1])
+    held.resident_tables().err[0] = 1
+    with pytest.raises(N.NativeError, match="waited too long"):
+        held.check()
+    with pytest.raises(RuntimeError, match="forward"):
+        held.migrate(res)  # the history went with the run
+    out = _gradient(held, res)
+    assert _same(out[0], ref[0]) and _same(out[1], ref[1])
+
+
+def test_modeling_raises_for_an_expired_wait(gpu, monkeypatch):
+    """forward_model raises in the call whose wait expired, and the next call
+    is right."""
+    import pysit_amd as pa
+    from pysit_amd import _native as N
+    from pysit_amd import resident
+    from tests.problems import c1_setup
+    m, shots, solver, model = c1_setup(tf=0.3)
+    ref = pa.TemporalModeling(solver, tile_x=8).forward_model(shots[0], model, return_parameters=["simdata"])
+    monkeypatch.setattr(resident, "SPIN", 1)
+    tools = pa.TemporalModeling(solver)
+    print("resident expired forward_model", flush=True)
+    with pytest.raises(N.NativeError, match="waited too long"):
+        tools.forward_model(shots[0], model, return_parameters=["simdata"])
+    out = tools.forward_model(shots[0], model, return_parameters=["simdata"])
+    assert np.array_equal(out["simdata"], ref["simdata"])
