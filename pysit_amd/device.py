@@ -832,8 +832,11 @@ class DeviceBatch:
 
     def resident_tables(self):
         """The tables of the resident loop, or None if this batch does not
-        use it."""
+        use it, or has not built them when the stream is under capture (they
+        are allocated and uploaded)."""
         if self._resident is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
             self._resident = ResidentTables.build(self, self._resident_always) or False
         return self._resident or None
 
@@ -848,10 +851,9 @@ class DeviceBatch:
             return None
         if mode == 2 and (not b.dw or bool(b.ic32) != (self.dtype == np.float32)):
             return None
-        tables = self.resident_tables()
-        if tables is None or torch.cuda.is_current_stream_capturing():
+        if torch.cuda.is_current_stream_capturing():
             return None
-        return tables
+        return self.resident_tables()
 
     def check(self):
         """Raise if a wait of the resident loop expired in a run whose results

@@ -85,3 +85,19 @@ def test_tables_cover_the_grid_and_stay_in_bounds(seed):
         for k in one:
             check_strip(plan, strips[k], R)
     assert held
+
+
+def test_a_capturing_stream_builds_no_tables(monkeypatch):
+    """Under capture a batch without resident tables takes the step kernels
+    and builds nothing; outside it asks for them again."""
+    import torch
+    from pysit_amd import _native, device
+    built = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(device.ResidentTables, "build", lambda batch, always: built.append(batch))
+    b = object.__new__(device.DeviceBatch)
+    b._resident, b._resident_always, b.persistent, b.dtype = None, False, False, np.dtype(np.float64)
+    assert b._resident_for(_native.Batch(), 0, 100) is None and b.resident_tables() is None
+    assert not built and b._resident is None
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    assert b.resident_tables() is None and built == [b]
