@@ -888,6 +888,8 @@ class DeviceBatch:
             ev[0].record()
         atp, arp = at.ctypes.data_as(ctypes.c_void_p), ar.ctypes.data_as(ctypes.c_void_p)
         resident = self._resident_for(b, mode, j1 - j0)
+        if resident is None and mode == 2 and b.inj_ptr:
+            self._precompute_sources(b, j1 - seg_base)
         if resident is not None:
             resident.run(self, b, mode, j0, j1, direction, seg_base, record, _stream())
         elif (self.persistent and self.dim == 2 and mode in (0, 1, 2) and not (b.dw_out or b.vol_dw)
@@ -1244,19 +1246,7 @@ class DeviceBatch:
             qb.ic32 = ic32.data_ptr()
             qb.ic_window = self.ic_window
             self._ic32 = ic32
-        # the adjoint sources of each run (the whole loop, or one checkpoint
-        # segment) are evaluated before its first step: a step then reads one
-        # value per node instead of gathering the node's receiver entries
-        n_nodes = int(self.adj_inj[2].numel()) - 1
-        # (the resident loop evaluates them itself, a chunk of slots at a time)
-        held = image and not (second or store_field or binomial) and self.dim == 2 and not self.persistent \
-            and (self.dtype == np.float64) != (ic32 is not None) and self.resident_tables() is not None
-        if n_nodes > 0 and self.precompute_injection and not held:
-            slots = K if ((self.ckpts or binomial) and image) else self.max_nt
-            qb.inj_pre = self._inj_pre_buffer(slots, n_nodes).data_ptr()
-            qb.inj_node_shot = self.adj_inj[5].data_ptr()
-            qb.n_inj_nodes = n_nodes
-            qb.inj_pre_slots = slots
+        qb.sweep_slots = K if ((self.ckpts or binomial) and image) else self.max_nt
         self.adjoint_store = None
         if store_field:
             self.adjoint_store = self._field_store()
@@ -1387,6 +1377,24 @@ class DeviceBatch:
         v = self._shot_view(self.dw_sq, self.order_idx.index(si_caller))
         sl = tuple(slice(l, n - r) for (l, r), n in zip(pads, v.shape))
         return v[sl]
+
+    def _precompute_sources(self, b, slots):
+        """Have the step kernels evaluate the adjoint sources of a run that
+        reaches ``slots`` slots past its store's base before its first step:
+        a step then reads one value per node instead of gathering the node's
+        receiver entries.  (The resident loop evaluates them itself, a chunk
+        of slots at a time.)  The buffer holds the longest run of the sweep,
+        so its address and size stay; of a batch that holds the other runs
+        on the chip, this run."""
+        n_nodes = int(self.adj_inj[2].numel()) - 1
+        if n_nodes == 0 or not self.precompute_injection:
+            return
+        if not self._resident:
+            slots = b.sweep_slots
+        b.inj_pre = self._inj_pre_buffer(slots, n_nodes).data_ptr()
+        b.inj_node_shot = self.adj_inj[5].data_ptr()
+        b.n_inj_nodes = n_nodes
+        b.inj_pre_slots = slots
 
     def _inj_pre_buffer(self, slots, n_nodes):
         """Device buffer for the precomputed injection of ``slots`` slots

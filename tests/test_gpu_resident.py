@@ -211,3 +211,14 @@ def test_modeling_raises_for_an_expired_wait(gpu, monkeypatch):
         tools.forward_model(shots[0], model, return_parameters=["simdata"])
     out = tools.forward_model(shots[0], model, return_parameters=["simdata"])
     assert np.array_equal(out["simdata"], ref["simdata"])
+
+
+def test_short_adjoint_segments_precompute_their_sources(gpu):
+    """An adjoint run too short for the resident loop reads its sources
+    precomputed, as every run of the step kernels does."""
+    p = Synthetic((60, 50), ((6, 6), (5, 5)), (0.01, 0.01), 97, 8, seed=3)
+    steps, held = _pair([p], np.float32)
+    ref = _gradient(steps, _residuals([p]))
+    out = _gradient(held, _residuals([p]), segment=30)
+    assert _same(out[0], ref[0]) and _same(out[1], ref[1])
+    assert held._inj_pre.numel() == 7 * (held.adj_inj[2].numel() - 1)  # slots 90 to 96
