@@ -207,7 +207,37 @@ def _split(total, rows, R):
     return [base + (i < extra) for i in range(n)]
 
 
-_LAYOUTS = {}
+class _Kept(object):
+    """At most ``most`` values by key, the one used longest ago dropped first;
+    several threads may ask at once (a value may then be made twice)."""
+
+    def __init__(self, most):
+        self.most = most
+        self._lock = threading.Lock()
+        self._kept = collections.OrderedDict()
+
+    def get(self, key, make):
+        with self._lock:
+            if key in self._kept:
+                self._kept.move_to_end(key)
+                return self._kept[key]
+        value = make()
+        with self._lock:
+            value = self._kept.setdefault(key, value)
+            self._kept.move_to_end(key)
+            while len(self._kept) > self.most:
+                self._kept.popitem(last=False)
+        return value
+
+    def clear(self):
+        with self._lock:
+            self._kept.clear()
+
+    def __len__(self):
+        return len(self._kept)
+
+
+_LAYOUTS = _Kept(4096)
 
 
 def _sorted_unique(a):
@@ -253,11 +283,7 @@ class ShotStrips(object):
         # columns each
         border = -(-self.nzc // 64) - (-full // 64)
         key = (nr, self.nzc - full, full, self.limits, border, self.R, alone)
-        if key not in _LAYOUTS:
-            if len(_LAYOUTS) > 4096:
-                _LAYOUTS.clear()
-            _LAYOUTS[key] = Layout(*key)
-        return _LAYOUTS[key]
+        return _LAYOUTS.get(key, lambda: Layout(*key))
 
     def costs(self, xtype):
         """(rows, cost) of the strips that fit a workgroup, by rows."""
@@ -414,7 +440,9 @@ def thread_items(lay, xtype, nzc, zfl, zfr, R, limits):
     return items, owner
 
 
-_PLANS = {}
+# a plan holds 0.1 to 0.6 MB; a survey of shots of uneven aperture,
+# modeled shot by shot, comes back to each of its plans (1.5 to 8 ms to make)
+_PLANS = _Kept(256)
 
 
 class Plan(object):
@@ -426,12 +454,7 @@ class Plan(object):
     @classmethod
     def of(cls, keys, R, itemsize, limits, cus):
         key = (keys, R, itemsize, limits, cus)
-        plan = _PLANS.get(key)
-        if plan is None:
-            if len(_PLANS) >= 32:
-                _PLANS.clear()
-            plan = _PLANS[key] = cls(*key)
-        return plan
+        return _PLANS.get(key, lambda: cls(*key))
 
     def __init__(self, keys, R, itemsize, limits, cus):
         groups = None

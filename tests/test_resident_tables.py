@@ -101,3 +101,41 @@ def test_a_capturing_stream_builds_no_tables(monkeypatch):
     assert not built and b._resident is None
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     assert b.resident_tables() is None and built == [b]
+
+
+def test_kept_plans_drop_one_at_a_time_and_serve_threads():
+    """Past its bound a store of plans drops the value used longest ago, not
+    all of them, and threads that fill and read it beyond the bound each get
+    the value of their key."""
+    import threading
+    kept = resident._Kept(4)
+    made = []
+    get = lambda k: kept.get(k, lambda: made.append(k) or ("plan", k))
+    for k in (0, 1, 2, 3, 0, 4, 0, 2):  # 1 goes when 4 comes
+        assert get(k) == ("plan", k)
+    assert made == [0, 1, 2, 3, 4] and len(kept) == 4
+    wrong = []
+
+    def work(seed):
+        rng = random.Random(seed)
+        for _ in range(3000):
+            k = rng.randrange(12)
+            if get(k) != ("plan", k):
+                wrong.append(k)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong and len(kept) == 4
+
+
+def test_a_survey_of_many_apertures_makes_each_plan_once(monkeypatch):
+    made = []
+    init = resident.Plan.__init__
+    monkeypatch.setattr(resident.Plan, "__init__", lambda self, *a: made.append(a[0]) or init(self, *a))
+    resident._PLANS.clear()
+    for _ in range(2):
+        for w in range(60, 100):
+            resident.Plan.of((((w, 60), ((6, 6), (5, 5)), 1),), 2, 4, LIMITS, 256)
+    assert len(made) == 40
