@@ -250,6 +250,11 @@ GRAPH_STEPS = 64
 RESIDENT_MIN_SLOTS = 8
 
 
+def by_length(shots):
+    """A batch's order of ``shots``: the longest first, else as given."""
+    return sorted(range(len(shots)), key=lambda i: -shots[i].nt)
+
+
 class DeviceBatch:
     """Tables and state of a shot batch on one GPU."""
 
@@ -345,6 +350,7 @@ class DeviceBatch:
         if resident is None:
             resident = not tile_x and graph_steps is None and tile_order == "shot"
         self._resident = None if resident else False  # False: never; None: tables not built yet
+        self._resident_plan = None                    # what the tables are built from, if it is known
 
         if isinstance(model, torch.Tensor):
             self.model = model.detach().to(device=self.dev, dtype=self.tdtype).contiguous()
@@ -358,7 +364,7 @@ class DeviceBatch:
 
         self.max_nt = max(s.nt for s in shots)
         kshift = [self.max_nt - s.nt for s in shots]
-        self.order_idx = sorted(range(len(shots)), key=lambda i: kshift[i])  # stable
+        self.order_idx = by_length(shots)
         self.shots = [shots[i] for i in self.order_idx]
         self.kshift = [kshift[i] for i in self.order_idx]
         self.n_shots = len(self.shots)

@@ -27,7 +27,8 @@ import numpy as np
 
 from .._native import NativeError
 from ..core.receivers import adjoint_entries, sampling_entries
-from ..device import DeviceBatch, ShotGeometry
+from ..device import DeviceBatch, ShotGeometry, _dev, by_length
+from ..resident import ResidentTables
 
 __all__ = ["TemporalModeling", "DWaveOpHandle"]
 
@@ -160,11 +161,13 @@ class TemporalModeling(object):
         if self._step_kernels:
             kw["resident"] = False
         if self.autotune and not self.tile_x:
-            if s.mesh.dim == 2:
-                b = DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
-                if b.resident_tables() is not None:
-                    return b  # its loop has no launch configuration to tune
-                del b
+            if s.mesh.dim == 2 and not self._step_kernels:
+                plan = ResidentTables.plan([geometries[i] for i in by_length(geometries)],
+                                           s.spatial_accuracy_order // 2, np.dtype(s.dtype).itemsize, _dev())
+                if plan is not None:  # its loop has no launch configuration to tune
+                    b = DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
+                    b._resident_plan = plan
+                    return b
             from ..autotune import tuned_batch
             return tuned_batch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, **kw)
         return DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, tile_x=self.tile_x,

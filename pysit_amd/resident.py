@@ -515,17 +515,19 @@ class ResidentTables(object):
     None where the batch does not suit it)."""
 
     @classmethod
-    def build(cls, batch, always=False):
+    def plan(cls, shots, R, item, dev, always=False):
+        """The plan of a batch of ``shots`` in its own order (``by_length``),
+        or None where the step kernels take it: known before any table or
+        state of the batch is made."""
         import torch
-        if batch.dim != 2 or batch.adj_inj is None:
+        if not shots or R not in (1, 2, 3, 4) or not all(cls._plannable(s) for s in shots):
             return None
         limits = N.resident_limits()
-        item = batch.dtype.itemsize
-        most = cls._source_cells_per_row(batch.shots, 16 // item)
+        most = cls._source_cells_per_row(shots, 16 // item)
         keys = tuple((tuple(int(n) for n in s.shape), tuple((l.size, r.size) for l, r in s.kpml), int(m))
-                     for s, m in zip(batch.shots, most))
-        cus = torch.cuda.get_device_properties(batch.dev).multi_processor_count
-        plan = Plan.of(keys, batch.R, item, limits, cus)
+                     for s, m in zip(shots, most))
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        plan = Plan.of(keys, R, item, limits, cus)
         if not plan.ok:
             return None
         # few nodes in costly strips (thick PML, FP64 of order 8) step faster
@@ -535,7 +537,25 @@ class ResidentTables(object):
         nodes = sum(k[0][0] * k[0][1] for k in keys)
         if not always and plan.cost > STEP_KERNEL_COST + nodes * item / STEP_KERNEL_BYTES:
             return None
-        return cls(batch, plan, limits)
+        return plan
+
+    @classmethod
+    def build(cls, batch, always=False):
+        """The tables of ``batch``, from its plan if the batch was made with
+        one."""
+        plan = batch._resident_plan
+        if plan is None:
+            plan = cls.plan(batch.shots, batch.R, batch.dtype.itemsize, batch.dev, always)
+        return None if plan is None else cls(batch, plan, N.resident_limits())
+
+    @staticmethod
+    def _plannable(s):
+        """Whether shot ``s`` is 2D with adjoint entries and every entry lies
+        on its grid (a batch refuses those that do not)."""
+        if len(s.shape) != 2 or s.adj is None:
+            return False
+        return all(e[0].shape[0] == 0 or (e[0].min() >= 0 and np.all(e[0].max(axis=0) < s.shape))
+                   for e in (s.src, s.adj))
 
     @staticmethod
     def _source_cells_per_row(shots, V):

@@ -139,3 +139,42 @@ def test_a_survey_of_many_apertures_makes_each_plan_once(monkeypatch):
         for w in range(60, 100):
             resident.Plan.of((((w, 60), ((6, 6), (5, 5)), 1),), 2, 4, LIMITS, 256)
     assert len(made) == 40
+
+
+class _Device(object):
+    multi_processor_count = 256
+
+
+@pytest.mark.parametrize("shape,pml,dtype,held", [((77, 67), 8, np.float32, True), ((116, 288), 50, np.float64, False)])
+def test_a_batch_is_built_once_whichever_loop_takes_it(monkeypatch, shape, pml, dtype, held):
+    """The route is known from the shots' sizes: neither loop's batch is made
+    only to be thrown away, and an entry outside the grid reaches the check
+    that refuses it."""
+    import types
+    import torch
+    from pysit_amd import autotune
+    from pysit_amd.modeling import temporal_modeling as tmod
+    from tests.problems import Synthetic
+    made = []
+
+    class Batch(object):
+        def __init__(self, *a, **kw):
+            made.append("resident")
+
+    monkeypatch.setattr(resident.N, "resident_limits", lambda: LIMITS)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda dev: _Device)
+    monkeypatch.setattr(tmod, "DeviceBatch", Batch)
+    monkeypatch.setattr(autotune, "tuned_batch", lambda *a, **kw: made.append("steps"))
+    mesh = types.SimpleNamespace(dim=2, deltas=(0.01, 0.01))
+    solver = types.SimpleNamespace(supports={"equation_dynamics": "time"}, mesh=mesh, dt=1e-3, dtype=dtype,
+                                   spatial_accuracy_order=8)
+    tools = tmod.TemporalModeling(solver)
+    g = Synthetic(shape, ((pml, pml), (pml, pml)), (0.01, 0.01), 20, 8).geometry()
+    tools.make_batch([g], None)
+    assert made == (["resident"] if held else ["steps"])
+    del made[:]
+    g.src[0][0] = shape[0], 3
+    tools.make_batch([g], None)
+    assert made == ["steps"]  # whose batch refuses the entry
