@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from . import _native as N
-from .resident import ResidentTables
+from .resident import RESIDENT_MIN_SLOTS, ResidentTables
 
 TILE_Z = 64      # z nodes per wavefront (the contiguous axis)
 
@@ -245,9 +245,6 @@ GRAPH_MAX_NODES = 1 << 20
 # default graph chunk, a multiple of it so that graph chunks hold whole windows
 IC_WINDOW = 64
 GRAPH_STEPS = 64
-# shorter runs than this many slots go through the step kernels: a resident
-# launch loads and stores the whole state
-RESIDENT_MIN_SLOTS = 8
 
 
 def by_length(shots):
@@ -918,21 +915,47 @@ class DeviceBatch:
 
         The store needs K * total_n values, the adjoint's precomputed
         sources K values per injection node; each checkpoint keeps the whole
-        state.  K is the largest value whose store plus checkpoints fit the
-        memory budget (default: 90% of the memory available to this batch:
-        free device memory, memory torch holds unused, and this batch's own
-        store and checkpoints, which a new run reuses or releases)."""
+        state, and the resident loop has buffers of its own.  K is the
+        largest value whose store plus checkpoints fit the memory budget
+        (default: 90% of the memory available to this batch: free device
+        memory, memory torch holds unused, and this batch's own store and
+        checkpoints, which a new run reuses or releases).  Where a budget
+        holds a cheaper schedule without the resident loop's buffers (nested
+        checkpoints instead of the binomial schedule, or any at all), the
+        batch goes on with the step kernels."""
         self.snaps = None
         if not keep_dw:
             return self.max_nt
         if self.schedule not in ("auto", "binomial"):
             raise ValueError("schedule must be 'auto' or 'binomial'")
+        tables = self.resident_tables()
+        if not tables:
+            return self._plan_budget(None)
+        try:
+            K = self._plan_budget(tables)
+            if self.schedule == "binomial" or self.snaps is None:
+                return K
+            plan = K, self.levels, self.snaps
+        except MemoryError:
+            plan = None
+        K = self._plan_budget(None)
+        if plan is not None and self.snaps is not None:
+            K, self.levels, self.snaps = plan
+        else:
+            self._resident = False
+        return K
+
+    def _plan_budget(self, tables):
+        """``plan_segments`` with the buffers of the resident loop's
+        ``tables`` counted, or without the loop."""
+        self.snaps = None
         budget = self.memory_budget
         item = self.dtype.itemsize
         n_inj = int(self.adj_inj[2].numel()) - 1 if self.adj_inj is not None else 0
         per_slot = (self.total_n + n_inj) * item
         ckpt = self.ckpt_bytes()
         state = self.state_bytes()
+        loop = tables.reserve(self.max_nt, budget) if tables else 0
         if budget is None:
             # everything this batch holds from an earlier gradient counts as
             # available (a new one reuses or releases it), so repeated calls
@@ -944,11 +967,12 @@ class DeviceBatch:
             mine += [v for c in getattr(self, "ckpts", []) for v in c.values()]
             held = sum(v.numel() * v.element_size() for v in mine if v is not None)
             held += state if getattr(self, "qstate", None) is not None else 0
+            held += tables.held() if tables else 0
             budget = int(0.9 * (free + unused + held))
         # what migrate allocates beside the store: the adjoint state, the
         # working state of the replays and the FP64 and FP32 imaging
         # accumulators
-        budget -= state + 12 * self.total_n
+        budget -= state + 12 * self.total_n + loop
         self.levels = [self.max_nt]
         self.snaps = None
         if self.schedule == "binomial":

@@ -40,8 +40,15 @@ SHARE_COST = 1.0
 # and the bytes of one field that add 1
 STEP_KERNEL_COST = 35.0
 STEP_KERNEL_BYTES = 30000.0
-# device memory for the source values and receiver nodes of a chunk of slots
+# device memory for the source values and receiver nodes of a chunk of slots,
+# and its part of a memory budget that a caller sets: 1/16 of 4 GB holds 700
+# slots of 16 shots of 1041 x 341 nodes, and a launch more per 100 slots costs
+# such a batch 1 %
 CHUNK_BYTES = 256 << 20
+CHUNK_SHARE = 16
+# shorter runs than this many slots go through the step kernels: a resident
+# launch loads and stores the whole state
+RESIDENT_MIN_SLOTS = 8
 # polls of about 1 us (16 s) before a wait for a neighbour gives up: a strip
 # may start late where another stream's kernels hold compute units
 SPIN = 1 << 24
@@ -636,7 +643,8 @@ class ResidentTables(object):
         stride = 2 * limits[4] * 4 + 4 * cells * 16
         self.xchg = torch.zeros(n * stride // 4, dtype=torch.int32, device=dev)
         self.epoch = ctypes.c_uint(0)
-        self._work = None
+        self._work, self._item = None, item
+        self._slot_bytes = (max(1, max(self.n_inj)) + max(1, self.n_rec_nodes)) * item
         q = self.struct = N.Resident()
         q.n_strips, q.n_groups = n, len(self.group_lds)
         q.group_begin = self.group_begin.ctypes.data
@@ -689,14 +697,36 @@ class ResidentTables(object):
         return {"lds": lds, "nptr": np.append(first, pos.size), "chan": chan, "w": w, "shot": shot[first],
                 "finfo": finfo, "cells": np.diff(begin)}
 
+    def chunk_slots(self, max_nt, budget):
+        """Slots of a run of ``max_nt`` that are worked on at a time: what
+        CHUNK_BYTES, or the working space's share of a memory ``budget`` if
+        there is one, hold of source values and receiver nodes, and 32 or 8
+        at least."""
+        room, least = CHUNK_BYTES, 32
+        if budget is not None:
+            room, least = min(CHUNK_BYTES, int(budget) // CHUNK_SHARE), RESIDENT_MIN_SLOTS
+        return min(max_nt, max(least, room // self._slot_bytes))
+
+    def reserve(self, max_nt, budget):
+        """Bytes that the loop takes beside the batch's state and stores in
+        runs of up to ``max_nt`` slots: tables, border rows, working space,
+        and the sources of a run too short for the loop."""
+        short = max(self.n_inj) * min(max_nt, RESIDENT_MIN_SLOTS - 1) * self._item
+        return (self._tables.numel() + self.xchg.numel()) * 4 + self._slot_bytes * self.chunk_slots(max_nt, budget) \
+            + short
+
+    def held(self):
+        """Bytes of what ``reserve`` counts that are allocated."""
+        return (self._tables.numel() + self.xchg.numel()) * 4 + (self._work[0] * self._slot_bytes if self._work else 0)
+
     def _workspace(self, batch):
         """Source values and receiver nodes of a chunk of slots."""
         import torch
-        if self._work is None or self._work[0] < min(batch.max_nt, self._chunk):
-            item = batch.dtype.itemsize
-            per_slot = (max(self.n_inj) + self.n_rec_nodes + 1) * item
-            self._chunk = max(32, CHUNK_BYTES // per_slot)
-            slots = min(batch.max_nt, self._chunk)
+        slots = self.chunk_slots(batch.max_nt, batch.memory_budget)
+        have = self._work[0] if self._work else 0
+        # a larger one stays where nothing bounds it (the time axis may change again)
+        if have < slots or (have > slots and batch.memory_budget is not None):
+            self._work = None  # first: both together may not fit
             pre = torch.empty(slots * max(1, max(self.n_inj)), dtype=batch.tdtype, device=batch.dev)
             rec = torch.empty(slots * max(1, self.n_rec_nodes), dtype=batch.tdtype, device=batch.dev)
             self._work = (slots, pre, rec)

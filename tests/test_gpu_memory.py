@@ -32,3 +32,31 @@ def test_repeated_forward_keeps_the_whole_history(gpu, monkeypatch):
     b.memory_budget = store * 6 // 10
     b.forward(keep_dw=True)
     assert b.K < b.max_nt and len(b.ckpts) >= 2
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("part", [0.3, 0.6, 1.3])
+def test_budget_bounds_a_gradient_on_the_resident_loop(gpu, dtype, part):
+    """What a gradient allocates beside the forward state and the tables that
+    a batch is built with stays within its budget, stored whole or by
+    checkpoints, and the loop is still what runs it."""
+    import torch
+    from pysit_amd.device import DeviceBatch
+    probs = [Synthetic((333, 201), ((12, 12), (12, 12)), (0.01, 0.01), 400, 8, seed=s, n_rec=300) for s in range(2)]
+    for p in probs[1:]:
+        p.model, p.Cpad, p.dt = probs[0].model, probs[0].Cpad, probs[0].dt
+    rng = np.random.default_rng(0)
+    res = [torch.from_numpy(rng.standard_normal((p.nt, p.n_rec))).cuda() for p in probs]
+    b = DeviceBatch([p.geometry() for p in probs], probs[0].model, probs[0].deltas, probs[0].dt, 8, dtype=dtype,
+                    resident=True)
+    budget = b.memory_budget = int(part * 400 * b.total_n * b.dtype.itemsize)
+    torch.cuda.synchronize()
+    # bytes asked for: the allocator may serve each from a block up to 1 MiB larger
+    asked = lambda which: torch.cuda.memory_stats()["requested_bytes.all." + which]
+    before = asked("current")
+    torch.cuda.reset_peak_memory_stats()
+    for _ in range(2):
+        b.forward(keep_dw=True)
+        b.migrate(res)
+        assert asked("peak") - before <= budget
+    assert b._resident and (not b.ckpts) == (part > 1)

@@ -178,3 +178,53 @@ def test_a_batch_is_built_once_whichever_loop_takes_it(monkeypatch, shape, pml, 
     g.src[0][0] = shape[0], 3
     tools.make_batch([g], None)
     assert made == ["steps"]  # whose batch refuses the entry
+
+
+class _Loop(object):
+    """Resident tables that take ``size`` bytes."""
+
+    def __init__(self, size):
+        self.size = size
+
+    def reserve(self, max_nt, budget):
+        return self.size
+
+    def held(self):
+        return 0
+
+
+@pytest.mark.parametrize("loop", [0, 1000, 40000, 10 ** 9])
+def test_a_memory_budget_counts_the_loop(loop):
+    """The schedule leaves room for the loop's buffers; where they would cost
+    a level of the schedule's kind or all of it, the batch does without them,
+    and a budget that held a schedule before still does."""
+    import torch
+    from pysit_amd import device
+    nt, n, nodes = 200, 1000, 30
+
+    def batch(budget, tables):
+        b = object.__new__(device.DeviceBatch)
+        b._resident, b.schedule, b.memory_budget, b.max_snaps = tables, "auto", budget, None
+        b.dtype, b.dim, b.total_n, b.max_nt = np.dtype(np.float32), 2, n, nt
+        b.adj_inj = (None, None, torch.zeros(nodes + 1))
+        return b
+
+    state, ckpt, slot = 7 * n * 4, 4 * n * 4, (n + nodes) * 4
+    for budget in range(state + 12 * n + 60000, state + 12 * n + nt * slot + 20000, 7777):
+        plain = batch(budget, False)
+        try:
+            K = plain.plan_segments(True)
+        except MemoryError:
+            continue
+        b = batch(budget, _Loop(loop))
+        Kb = b.plan_segments(True)
+        size = loop if b._resident else 0
+        assert (plain.snaps is None) == (b.snaps is None)
+        if b.snaps is None:
+            levels = b.levels if Kb < nt else []
+            counts = [-(-a // k) for a, k in zip([nt] + levels, levels)]
+            stored = (levels or [nt])[-1]
+            need = stored * slot + sum(counts) * ckpt + (state if levels else 0)
+            assert need + size + state + 12 * n <= budget
+            if not b._resident:
+                assert Kb == K and b.levels == plain.levels and loop > 0
