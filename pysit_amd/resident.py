@@ -461,7 +461,8 @@ class Plan(object):
     @classmethod
     def of(cls, keys, R, itemsize, limits, cus):
         key = (keys, R, itemsize, limits, cus)
-        return _PLANS.get(key, lambda: cls(*key))
+        # with the rule that groups the shots: a plan is kept for it alone
+        return _PLANS.get((plan_groups,) + key, lambda: cls(*key))
 
     def __init__(self, keys, R, itemsize, limits, cus):
         groups = None

@@ -228,3 +228,14 @@ def test_a_memory_budget_counts_the_loop(loop):
             assert need + size + state + 12 * n <= budget
             if not b._resident:
                 assert Kb == K and b.levels == plain.levels and loop > 0
+
+
+def test_a_kept_plan_belongs_to_its_grouping(monkeypatch):
+    """Another rule that groups the shots makes its own plan, whatever is kept
+    from an earlier one."""
+    keys = (((61, 53), ((6, 7), (5, 8)), 1),) * 3
+    one = resident.Plan.of(keys, 4, 8, LIMITS, 256)
+    rule = resident.plan_groups
+    monkeypatch.setattr(resident, "plan_groups", lambda shots, cus: rule(shots, len(shots[0].cut(1e9))))
+    other = resident.Plan.of(keys, 4, 8, LIMITS, 256)
+    assert len(one.group_begin) == 2 and len(other.group_begin) > 2
