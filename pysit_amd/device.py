@@ -247,6 +247,51 @@ IC_WINDOW = 64
 GRAPH_STEPS = 64
 
 
+_TORCH = {np.dtype(np.int32): torch.int32, np.dtype(np.int64): torch.int64, np.dtype(np.float64): torch.float64}
+
+
+def _same_memory(*arrays):
+    """A key of arrays within one call: equal keys are the same elements."""
+    return tuple((a.__array_interface__["data"][0], a.shape, a.strides) for a in arrays)
+
+
+class NodeEntries:
+    """Entries (flat node, channel, weight) gathered by node: the ``node``s in
+    ascending order, each with its entries [nptr[i], nptr[i + 1]) of ``chan``
+    and ``w`` in the order they were given in."""
+
+    def __init__(self, flat, chan, w):
+        if min(chan.size, w.size) < flat.size:
+            raise IndexError("an entry without its channel or weight")
+        self.given, self._order, chan, w = flat, None, chan[:flat.size], w[:flat.size]
+        if np.any(flat[1:] < flat[:-1]):
+            self._order = np.argsort(flat, kind="stable")
+            flat, chan, w = flat[self._order], chan[self._order], w[self._order]
+        self._starts = np.ones(flat.size, dtype=bool)
+        np.not_equal(flat[1:], flat[:-1], out=self._starts[1:])
+        first = np.flatnonzero(self._starts)
+        self.node = flat[first]
+        self.nptr = np.append(first, flat.size)
+        self.chan, self.w = chan.astype(np.int32), np.ascontiguousarray(w)
+
+    def rank(self):
+        """The node (its number) of every given entry."""
+        r = np.cumsum(self._starts, dtype=np.int32) - np.int32(1)
+        if self._order is None:
+            return r
+        out = np.empty_like(r)
+        out[self._order] = r
+        return out
+
+
+def reordered(perm, nptr, *arrays):
+    """(nptr, arrays) of the nodes taken in order ``perm``, entries with them."""
+    count = np.diff(nptr)[perm]
+    new = np.concatenate([[0], np.cumsum(count)])
+    entry = np.repeat(nptr[perm] - new[:-1], count) + np.arange(new[-1])
+    return (new,) + tuple(a[entry] for a in arrays)
+
+
 def by_length(shots):
     """A batch's order of ``shots``: the longest first, else as given."""
     return sorted(range(len(shots)), key=lambda i: -shots[i].nt)
@@ -451,7 +496,9 @@ class DeviceBatch:
         # (zs >= nz; the nodes past nz are never read or written)
         self.offs, self.zs, self.snpts = [], [], []
         off = 0
-        tiles_info = []
+        # (alike shots share their tiles, and the entries of one operator are
+        # gathered once: a survey's tables cost what those of one shot do)
+        tiles_info, known = [], {}
         for s in self.shots:
             nz = s.shape[-1]
             zs = -(-nz // self.zalign) * self.zalign
@@ -460,7 +507,10 @@ class DeviceBatch:
             self.zs.append(zs)
             self.snpts.append(sn)
             off += sn
-            tiles_info.append(self._tiles_of(s))
+            like = (s.shape, tuple((l.size, r.size) for l, r in s.kpml))
+            if like not in known:
+                known[like] = self._tiles_of(s)
+            tiles_info.append(known[like])
         self.total_n = off
         limit = max_batch_nodes(self.dim, self.dtype.itemsize)
         if off > limit:
@@ -472,61 +522,55 @@ class DeviceBatch:
         # else shot-major (active prefix by kshift)
         same = all(s.shape == self.shots[0].shape and s.window == self.shots[0].window
                    for s in self.shots) and len(set(self.kshift)) == 1 and self.tile_order == "interleave"
-        rows = []
-        # column 3: the x tile index, t // (tiles per x row)
-        per_x = [ti[0][1] * ti[0][2] for ti in tiles_info]
-        if same:
-            ntile = len(tiles_info[0][1])
-            for t in range(ntile):
-                for si in range(self.n_shots):
-                    rows.append((si, t, int(tiles_info[si][1][t]), t // per_x[si]))
-        else:
-            for si in range(self.n_shots):
-                fl = tiles_info[si][1]
-                for t in range(len(fl)):
-                    rows.append((si, t, int(fl[t]), t // per_x[si]))
-        tiles = np.asarray(rows, dtype=np.int32).reshape(-1, 4)
+        # rows {shot, tile in it, flags, x tile: t // (tiles per x row)}
+        count = [len(ti[1]) for ti in tiles_info]
+        rows = [np.stack([np.full(n, si), np.arange(n), ti[1], np.arange(n) // (ti[0][1] * ti[0][2])], axis=1)
+                for si, (n, ti) in enumerate(zip(count, tiles_info))]
+        tiles = np.stack(rows, axis=1) if same else np.concatenate(rows)
+        tiles = tiles.reshape(-1, 4)
         self.n_tiles = tiles.shape[0]
-        # global tile id of (shot, tile within the shot): one lookup array per shot
-        self._tile_lookup = []
-        for si in range(self.n_shots):
-            look = np.full(len(tiles_info[si][1]), -1, dtype=np.int64)
-            mine = tiles[:, 0] == si
-            look[tiles[mine, 1]] = np.nonzero(mine)[0]
-            self._tile_lookup.append(look)
-        self.tiles = torch.from_numpy(tiles.reshape(-1).copy()).to(dev)
+        # tile id = first tile of the shot + stride * tile in the shot
+        self._tile_first = np.arange(self.n_shots) if same else np.cumsum([0] + count)[:-1]
+        self._tile_stride = self.n_shots if same else 1
 
         self._same = same
         self._active_prefix()
 
         # PML arrays and model windows (shared tensors where equal)
         self._keep = []
-        self.fwd_inj = self._injection_tables([s.src for s in self.shots])
+        # (by_node: each shot's nodes are in ascending order in the tables)
+        src, self.src_nodes, self.src_by_node = self._injection_tables([s.src for s in self.shots])
         has_adj = all(s.adj is not None for s in self.shots)
-        self.adj_inj = self._injection_tables([s.adj for s in self.shots]) if has_adj else None
+        adj, self.adj_nodes, self.adj_by_node = \
+            self._injection_tables([s.adj for s in self.shots]) if has_adj else ([], None, False)
 
-        # receivers
-        recs, ridx, rw = [], [], []
-        self._rec_sorted = []  # per shot, the entries' flat padded nodes in rec_w's order
-        e = 0
+        # receivers: entries by receiver, in the order they were given in
+        known, mine, recs, e = {}, [], [], 0
         for si, s in enumerate(self.shots):
-            idx, chan, w = s.rec
-            nz = s.shape[-1]
-            idx = (np.asarray(idx, dtype=np.int64) // nz) * self.zs[si] + np.asarray(idx, dtype=np.int64) % nz
-            order = np.argsort(chan, kind="stable")
-            idx, chan, w = idx[order], chan[order], w[order]
-            self._rec_sorted.append((idx // self.zs[si]) * nz + idx % self.zs[si])
-            counts = np.bincount(chan, minlength=s.nrec)
-            starts = np.concatenate([[0], np.cumsum(counts)])
-            for r in range(s.nrec):
-                recs.append((si, r, e + starts[r], e + starts[r + 1]))
-            ridx.append(idx)
-            rw.append(w)
-            e += idx.size
+            key = _same_memory(*s.rec) + (s.nrec, s.shape[-1])
+            if key not in known:
+                idx, chan, w = s.rec
+                if min(idx.size, w.size) < chan.size:
+                    raise IndexError("a receiver entry without its node or weight")
+                idx, w = idx[:chan.size], w[:chan.size]
+                if np.any(chan[1:] < chan[:-1]):
+                    order = np.argsort(chan, kind="stable")
+                    idx, chan, w = idx[order], chan[order], w[order]
+                x, z = np.divmod(idx, s.shape[-1])
+                ends = np.cumsum(np.bincount(chan, minlength=s.nrec))[:s.nrec]
+                known[key] = (idx, x * self.zs[si] + z, w, np.concatenate([[0], ends[:-1]])[:s.nrec], ends)
+            got = known[key]
+            mine.append(got)
+            recs.append(np.stack([np.full(s.nrec, si), np.arange(s.nrec), e + got[3], e + got[4]], axis=1))
+            e += got[0].size
+        # per shot, the entries' nodes (flat, unpadded rows) in rec_w's order
+        self.rec_nodes = [got[0] for got in mine]
+        recs = np.concatenate(recs)
         self.n_rec = len(recs)
-        self.recs = torch.from_numpy(np.asarray(recs, dtype=np.int32).reshape(-1)).to(dev)
-        self.rec_idx = torch.from_numpy(np.concatenate(ridx).astype(np.int64) if ridx else np.zeros(0, np.int64)).to(dev)
-        self.rec_w = torch.from_numpy(np.concatenate(rw) if rw else np.zeros(0)).to(dev)
+        sent = self._send(src + adj + [(np.int32, [tiles.reshape(-1)]), (np.int32, [recs.reshape(-1)]),
+                                       (np.int64, [got[1] for got in mine]), (np.float64, [got[2] for got in mine])])
+        self.fwd_inj, self.adj_inj = tuple(sent[:6]), tuple(sent[6:-4]) if has_adj else None
+        self.tiles, self.recs, self.rec_idx, self.rec_w = sent[-4:]
 
         # per-shot device arrays
         self.pml_dev = []
@@ -637,52 +681,83 @@ class DeviceBatch:
         if self._mz is not None:
             self.model_k.copy_(self._kernel_layout(self.model))
 
+    def _send(self, groups):
+        """Device tensors of several tables, in one copy (each costs some 25
+        us): per group a dtype and the host arrays it joins, of which one that
+        occurs more than once is sent once."""
+        size, made = 0, []
+        for dtype, arrays in groups:
+            begin, where = size, {}
+            for a in arrays:
+                if id(a) not in where:
+                    where[id(a)] = ((size - begin) // np.dtype(dtype).itemsize, a)
+                    size += a.size * np.dtype(dtype).itemsize
+            made.append((np.dtype(dtype), arrays, where, begin, size))
+            size += -size % 16
+        host = np.empty(size, dtype=np.uint8)
+        for dtype, _, where, begin, end in made:
+            to = host[begin:end].view(dtype)
+            for first, a in where.values():
+                to[first:first + a.size] = a
+        sent, out = torch.from_numpy(host).to(self.dev), []
+        for dtype, arrays, where, begin, end in made:
+            t = sent[begin:end].view(_TORCH[dtype])
+            if len(where) < len(arrays):
+                t = torch.cat([t[where[id(a)][0]:where[id(a)][0] + a.size] for a in arrays])
+            out.append(t)
+        return out
+
     def _injection_tables(self, entries):
         """Two-level CSR: tiles -> destination nodes -> entries.  Entries of
         one node keep the order they were given in (the order the reference's
         sparse product accumulates in).  Also the shot of every node (for the
-        precomputed injection)."""
-        node_tile, node_pos, node_key, e_chan, e_w, e_shot = [], [], [], [], [], []
+        precomputed injection).  Returns the tables as ``_send`` takes them, the
+        shots' :class:`NodeEntries` and whether every shot's nodes are in its
+        order."""
+        gathered, tiled = {}, {}
+        nodes, parts, in_order = [], [], True
         for si, (s, e) in enumerate(zip(self.shots, entries)):
             pos, chan, w = e
-            if pos.shape[0] == 0:
-                continue
-            if np.any(pos < 0) or np.any(pos >= np.asarray(s.shape)[None, :]):
-                raise ValueError("injection entry outside the padded grid")
-            tloc, local = self._tile_of_pos(s, self.tiles_info[si][0], pos)
-            tglob = self._tile_lookup[si][np.asarray(tloc, dtype=np.int64)]
-            node_tile.append(tglob)
-            node_pos.append(local)
-            e_chan.append(chan)
-            e_w.append(w)
-            e_shot.append(np.full(tglob.size, si, dtype=np.int32))
-        if node_tile:
-            tg = np.concatenate(node_tile)
-            lp = np.concatenate(node_pos)
-            ch = np.concatenate(e_chan)
-            wt = np.concatenate(e_w)
-            es = np.concatenate(e_shot)
-            order = np.lexsort((np.arange(tg.size), lp, tg))  # stable within a node
-            tg, lp, ch, wt, es = tg[order], lp[order], ch[order], wt[order], es[order]
-            key = tg * (1 << 20) + lp
-            starts = np.concatenate([[True], key[1:] != key[:-1]])
-            node_first = np.nonzero(starts)[0]
-            n_tile = tg[node_first]
-            n_pos = lp[node_first].astype(np.int32)
-            n_shot = es[node_first]
-            nptr = np.concatenate([node_first, [tg.size]]).astype(np.int32)
-            tcount = np.bincount(n_tile, minlength=self.n_tiles)
-        else:
-            n_pos = np.zeros(0, np.int32)
-            n_shot = np.zeros(0, np.int32)
-            nptr = np.zeros(1, np.int32)
-            ch = np.zeros(0, np.int64)
-            wt = np.zeros(0)
-            tcount = np.zeros(self.n_tiles, np.int64)
-        ptr = np.concatenate([[0], np.cumsum(tcount)]).astype(np.int32)
-        t = lambda a, dt: torch.from_numpy(np.ascontiguousarray(a, dtype=dt)).to(self.dev)
-        return (t(ptr, np.int32), t(n_pos, np.int32), t(nptr, np.int32), t(ch, np.int32), t(wt, np.float64),
-                t(n_shot, np.int32))
+            key = _same_memory(*e) + s.shape
+            if key not in gathered:
+                axes = [pos[:, i] for i in range(self.dim)]
+                if pos.shape[0] and any(a.min() < 0 or a.max() >= n for a, n in zip(axes, s.shape)):
+                    raise ValueError("injection entry outside the padded grid")
+                flat = axes[0]
+                for a, n in zip(axes[1:], s.shape[1:]):
+                    flat = flat * n + a
+                gathered[key] = NodeEntries(flat, chan, w)
+            ne = gathered[key]
+            nodes.append(ne)
+            if ne not in tiled:
+                at = np.stack(np.unravel_index(ne.node, s.shape), axis=1)
+                tile, local = self._tile_of_pos(s, self.tiles_info[si][0], at)
+                by_tile = tile * (1 << 20) + local
+                nptr, chan, w = ne.nptr, ne.chan, ne.w
+                if np.any(by_tile[1:] < by_tile[:-1]):
+                    perm = np.argsort(by_tile)
+                    tile, local = tile[perm], local[perm]
+                    nptr, chan, w = reordered(perm, nptr, chan, w)
+                    in_order = False
+                tiled[ne] = (tile, local.astype(np.int32), nptr, chan, w)
+            parts.append(tiled[ne])
+        count = [p[0].size for p in parts]
+        entry = np.cumsum([0] + [p[3].size for p in parts])
+        tile = np.concatenate([f + self._tile_stride * p[0] for f, p in zip(self._tile_first, parts)])
+        local = np.concatenate([p[1] for p in parts])
+        nptr = np.concatenate([e + p[2][:-1] for e, p in zip(entry, parts)] + [entry[-1:]])
+        shot = np.repeat(np.arange(self.n_shots, dtype=np.int32), count)
+        chan, w = [p[3] for p in parts], [p[4] for p in parts]
+        if np.any(tile[1:] < tile[:-1]):
+            # the shots of a tile follow one another
+            perm = np.argsort(tile, kind="stable")
+            tile, local, shot = tile[perm], local[perm], shot[perm]
+            nptr, *arrays = reordered(perm, nptr, np.concatenate(chan), np.concatenate(w))
+            chan, w = [arrays[0]], [arrays[1]]
+            in_order = False
+        ptr = np.concatenate([[0], np.cumsum(np.bincount(tile, minlength=self.n_tiles))])
+        i32, f64 = np.int32, np.float64
+        return ([(i32, [ptr]), (i32, [local]), (i32, [nptr]), (i32, chan), (f64, w), (i32, [shot])], nodes, in_order)
 
     def _shot_table(self, amps, namps):
         arr = (N.Shot * self.n_shots)()

@@ -193,12 +193,15 @@ def _border_first(groups):
     return groups[:1] + groups[:0:-1][:1] + groups[1:-1] if len(groups) > 2 else groups
 
 
+def _copy_bytes(nr, nzc, full, hc, R, n_fcells):
+    return (((nr + 2 * R) * (nzc + hc) + hc) * 16, (nr + 2 * R) * full * 16, (nr * (full + 2 * hc) + hc) * 16,
+            n_fcells * 16)
+
+
 def lds_copies(strips, hc, R, n_fcells):
     """Bytes of one copy of u, Phix, Phiz and the source cells of strips (an
     array of their numbers, or one strip's)."""
-    nr, nzc, full = strips.T[2], strips.T[21], strips.T[4] + strips.T[5]
-    return (((nr + 2 * R) * (nzc + hc) + hc) * 16, (nr + 2 * R) * full * 16, (nr * (full + 2 * hc) + hc) * 16,
-            n_fcells * 16)
+    return _copy_bytes(strips.T[2], strips.T[21], strips.T[4] + strips.T[5], hc, R, n_fcells)
 
 
 def lds_offsets(copies, nr, itemsize):
@@ -208,10 +211,10 @@ def lds_offsets(copies, nr, itemsize):
 
 
 def _split(total, rows, R):
-    """Row counts of equal strips of at most ``rows`` rows, each at least R."""
+    """(strips, rows, strips of one row more) of equal strips of at most
+    ``rows`` rows, each at least R."""
     n = max(1, min(-(-total // rows), total // R if total >= R else 1))
-    base, extra = divmod(total, n)
-    return [base + (i < extra) for i in range(n)]
+    return (n,) + divmod(total, n)
 
 
 class _Kept(object):
@@ -247,14 +250,6 @@ class _Kept(object):
 _LAYOUTS = _Kept(4096)
 
 
-def _sorted_unique(a):
-    """np.unique with the inverse, without the sort where none is needed."""
-    if a.size == 0 or np.all(a[1:] > a[:-1]):
-        return a, np.arange(a.size)
-    u, inv = np.unique(a, return_inverse=True)
-    return u, inv.reshape(-1)
-
-
 class ShotStrips(object):
     """The ways to cut one shot into strips of at most ``most`` rows: its
     column split and, for a bound on the cost of a step, the strips (x0, rows,
@@ -275,14 +270,12 @@ class ShotStrips(object):
             self.segments = [(0, self.nx, True)]
         else:
             self.segments = [(0, left, True), (left, self.nx - left - right, False), (self.nx - right, right, True)]
-        self._costs = {}
+        self._costs, self._ok, self._splits = {}, {}, {}
 
     def fits(self, nr, xtype):
-        fl, fr = (self.nzc, 0) if xtype else (self.zfl, self.zfr)
-        d = np.zeros(STRIP_INTS, dtype=np.int64)
-        d[[2, 4, 5, 21]] = nr, fl, fr, self.nzc
-        copies = lds_copies(d, self.hc, self.R, self.n_fcells_row * nr)
-        return lds_offsets(copies, nr, self.itemsize)[-1] + 32 <= LDS_BYTES
+        full = self.nzc if xtype else self.zfl + self.zfr
+        copies = _copy_bytes(nr, self.nzc, full, self.hc, self.R, self.n_fcells_row * nr)
+        return 2 * sum(copies) + -(-nr * 2 * self.itemsize // 16) * 16 + 32 <= LDS_BYTES
 
     def layout(self, nr, xtype, alone=False):
         full = self.nzc if xtype else self.zfl + self.zfr
@@ -305,26 +298,49 @@ class ShotStrips(object):
             self._costs[xtype] = out
         return self._costs[xtype]
 
-    def cut(self, bound, rows_z=None):
+    def split(self, bound, rows_z=None):
         """Strips that cost at most ``bound`` a step, or None: the fewest, but
-        those away from the x PML of about ``rows_z`` rows if that is given."""
+        those away from the x PML of about ``rows_z`` rows if that is given;
+        per segment (x0, x type, strips, rows, strips of one row more)."""
+        if (bound, rows_z) not in self._splits:
+            self._splits[bound, rows_z] = self._split(bound, rows_z)
+        return self._splits[bound, rows_z]
+
+    def _split(self, bound, rows_z):
         if self.fits(self.nx, True) and rows_z is None:
             lay = self.layout(self.nx, True, True)
             if lay.ok and lay.cost <= bound:
-                return [(0, self.nx, True)]
+                return [(0, True, 1, self.nx, 0)]
         out = []
         for x0, total, xtype in self.segments:
-            ok = {nr for nr, c in self.costs(xtype) if c <= bound}
-            given = rows_z is not None and not xtype
-            for rows in ([rows_z] if given else sorted(ok, reverse=True)):
-                parts = _split(total, rows, self.R)
-                if all(nr in ok for nr in parts):
+            if (xtype, bound) not in self._ok:
+                ok = [nr for nr, c in self.costs(xtype) if c <= bound]
+                self._ok[xtype, bound] = ok[::-1], set(ok)
+            order, ok = self._ok[xtype, bound]
+            for rows in ([rows_z] if rows_z is not None and not xtype else order):
+                n, nr, more = _split(total, rows, self.R)
+                if nr in ok and (not more or nr + 1 in ok):
                     break
             else:
                 return None
-            for nr in parts:
-                out.append((x0, nr, xtype))
-                x0 += nr
+            out.append((x0, xtype, n, nr, more))
+        return out
+
+    def count(self, bound, rows_z=None):
+        """The number of strips of ``split``, or None."""
+        got = self.split(bound, rows_z)
+        return None if got is None else sum(s[2] for s in got)
+
+    def cut(self, bound, rows_z=None):
+        """``split`` strip by strip, (x0, rows, x type), or None."""
+        got = self.split(bound, rows_z)
+        if got is None:
+            return None
+        out = []
+        for x0, xtype, n, nr, more in got:
+            for i in range(n):
+                out.append((x0, nr + (i < more), xtype))
+                x0 += out[-1][1]
         return out
 
     def bounds(self):
@@ -343,12 +359,6 @@ def plan_groups(shots, cus):
     bounds = sorted(set().union(*[s.bounds() for s in set(shots)]))
     if not bounds:
         return None
-    cuts = {}
-
-    def cut(s, *bound):
-        if (s, bound) not in cuts:
-            cuts[(s, bound)] = s.cut(*bound)
-        return cuts[(s, bound)]
 
     def fill(group):
         """(bound, rows away from the x PML): the least bound whose strips fit
@@ -359,8 +369,8 @@ def plan_groups(shots, cus):
         strips and 6.0 with 123; 186 x 113 of order 8, 4.9 with 24 and 6.0 with
         19; 360 x 332 of order 4, 4.4 with 180 and 5.3 with 83)."""
         def count(*bound):
-            c = [cut(shots[i], *bound) for i in group]
-            return cus + 1 if any(x is None for x in c) else sum(len(x) for x in c)
+            c = [shots[i].count(*bound) for i in group]
+            return cus + 1 if None in c else sum(c)
         lo, hi = 0, len(bounds) - 1
         if count(bounds[hi]) > cus:
             return None
@@ -377,10 +387,9 @@ def plan_groups(shots, cus):
                     return bounds[lo], rows
         return (bounds[lo],)
 
-    fewest = [cut(s, bounds[-1]) for s in shots]
-    if any(f is None or len(f) > cus for f in fewest):
+    weight = [s.count(bounds[-1]) for s in shots]
+    if any(f is None or f > cus for f in weight):
         return None
-    weight = [len(f) for f in fewest]
     total = sum(weight)
     best = None
     first = max(1, -(-total // cus))
@@ -392,7 +401,7 @@ def plan_groups(shots, cus):
         groups = [g for g in groups if g]
         got = [fill(g) for g in groups]
         if all(b is not None for b in got) and (best is None or sum(b[0] for b in got) < best[0]):
-            best = (sum(b[0] for b in got), [(g, [cut(shots[i], *b) for i in g]) for g, b in zip(groups, got)])
+            best = (sum(b[0] for b in got), [(g, [shots[i].cut(*b) for i in g]) for g, b in zip(groups, got)])
         if best is not None and n >= first + 2:
             break
     return best
@@ -480,14 +489,19 @@ class Plan(object):
         self.cost, groups = groups
         cuts = [memo[k] for k in keys]
         self.nzc = np.array([c.nzc for c in cuts])
-        strips, templates, row_strip = [], {}, []
-        self.group_begin, self.row_base = [0], []
-        n_rows = 0
+        strips, templates = [], {}
+        self.group_begin, self.first_strip = [0], []
+        # per shot, which of the distinct cuts it has, and of these the strip of
+        # every row: shots of one cut have the same strips
+        self.cut_of, self.row_strip, known = [], [], {}
         for shots, cut in groups:
             for si, parts in zip(shots, cut):
                 c = cuts[si]
-                self.row_base.append(n_rows)
-                n_rows += c.nx
+                self.first_strip.append(len(strips))
+                if (c, tuple(parts)) not in known:
+                    known[c, tuple(parts)] = len(known)
+                    self.row_strip.append(np.repeat(np.arange(len(parts)), [nr for _, nr, _ in parts]))
+                self.cut_of.append(known[c, tuple(parts)])
                 for i, (x0, nr, xtype) in enumerate(parts):
                     lay = c.layout(nr, xtype, len(parts) == 1)
                     key = (lay, xtype, c.nzc, c.zfl, c.zfr)
@@ -506,11 +520,9 @@ class Plan(object):
                     d[19:24] = me - 1 if up else -1, me + 1 if down else -1, c.nzc, me, lay.exchange
                     d[28] = templates[key][0]
                     strips.append(d)
-                    row_strip.append(np.full(nr, me))
             self.group_begin.append(len(strips))
         self.strips = np.array(strips, dtype=np.int64)
-        self.row_strip = np.concatenate(row_strip)
-        self.row_base = np.array(self.row_base)
+        self.first_strip.append(len(strips))
         tables = [t for _, t in templates.values()]
         self.items = np.stack([t[0] for t in tables])
         # owners of the cells of all templates, (thread, step) a cell
@@ -523,16 +535,16 @@ class ResidentTables(object):
     None where the batch does not suit it)."""
 
     @classmethod
-    def plan(cls, shots, R, item, dev, always=False):
+    def plan(cls, shots, R, item, dev, always=False, nodes=None):
         """The plan of a batch of ``shots`` in its own order (``by_length``),
         or None where the step kernels take it: known before any table or
         state of the batch is made."""
         import torch
-        if not shots or R not in (1, 2, 3, 4) or not all(cls._plannable(s) for s in shots):
+        most = cls._source_cells_per_row(shots, 16 // item, nodes)
+        if not most or R not in (1, 2, 3, 4):
             return None
         limits = N.resident_limits()
-        most = cls._source_cells_per_row(shots, 16 // item)
-        keys = tuple((tuple(int(n) for n in s.shape), tuple((l.size, r.size) for l, r in s.kpml), int(m))
+        keys = tuple((tuple(int(n) for n in s.shape), tuple((l.size, r.size) for l, r in s.kpml), m)
                      for s, m in zip(shots, most))
         cus = torch.cuda.get_device_properties(dev).multi_processor_count
         plan = Plan.of(keys, R, item, limits, cus)
@@ -542,8 +554,8 @@ class ResidentTables(object):
         # through the caches: 116 x 288 nodes in FP64 at cost 113 takes 11.1 us
         # here and 8.6 there, 104 x 104 (4 shots, cost 53) 10.9 and 9.2; at
         # cost 53, 448 x 175 in FP64 takes 11.8 and 12.0
-        nodes = sum(k[0][0] * k[0][1] for k in keys)
-        if not always and plan.cost > STEP_KERNEL_COST + nodes * item / STEP_KERNEL_BYTES:
+        size = sum(k[0][0] * k[0][1] for k in keys)
+        if not always and plan.cost > STEP_KERNEL_COST + size * item / STEP_KERNEL_BYTES:
             return None
         return plan
 
@@ -553,33 +565,37 @@ class ResidentTables(object):
         one."""
         plan = batch._resident_plan
         if plan is None:
-            plan = cls.plan(batch.shots, batch.R, batch.dtype.itemsize, batch.dev, always)
+            plan = cls.plan(batch.shots, batch.R, batch.dtype.itemsize, batch.dev, always,
+                            (batch.src_nodes, batch.adj_nodes))
         return None if plan is None else cls(batch, plan, N.resident_limits())
 
     @staticmethod
-    def _plannable(s):
-        """Whether shot ``s`` is 2D with adjoint entries and every entry lies
-        on its grid (a batch refuses those that do not)."""
-        if len(s.shape) != 2 or s.adj is None:
-            return False
-        return all(e[0].shape[0] == 0 or (e[0].min() >= 0 and np.all(e[0].max(axis=0) < s.shape))
-                   for e in (s.src, s.adj))
-
-    @staticmethod
-    def _source_cells_per_row(shots, V):
+    def _source_cells_per_row(shots, V, nodes=None):
         """Per shot, the most source cells in any of its rows, forward or
-        adjoint."""
-        most = np.zeros(len(shots), dtype=np.int64)
-        nx, nz = (max(s.shape[i] for s in shots) for i in range(2))
-        cells = -(-nz // V)
-        for way in range(2):
-            pos = [(s.src, s.adj)[way][0] for s in shots]
-            si = np.repeat(np.arange(len(shots)), [p.shape[0] for p in pos])
-            if si.size:
-                pos = np.concatenate(pos)
-                some = np.zeros(len(shots) * nx * cells, dtype=bool)
-                some[(si * nx + pos[:, 0]) * cells + pos[:, 1] // V] = True
-                most = np.maximum(most, some.reshape(len(shots), nx, cells).sum(axis=2, dtype=np.int32).max(axis=1))
+        adjoint; None if one is not 2D, has no adjoint entries or has an entry
+        off its grid (which a batch refuses).  ``nodes``: per way and shot the
+        entries' flat nodes, where a batch has gathered them."""
+        known, most = {}, []
+        for si, s in enumerate(shots):
+            if len(s.shape) != 2 or s.adj is None:
+                return None
+            nx, nz = s.shape
+            cells = -(-nz // V)
+            n = 0
+            for way, (pos, _, _) in enumerate((s.src, s.adj)):
+                key = (pos.__array_interface__["data"][0], pos.shape, pos.strides, nx, nz)
+                if key not in known:
+                    known[key] = 0
+                    if pos.shape[0]:
+                        x, z = np.divmod(nodes[way][si].node, nz) if nodes else (pos[:, 0], pos[:, 1])
+                        x0, x1 = int(x.min()), int(x.max())
+                        if x0 < 0 or x1 >= nx or z.min() < 0 or z.max() >= nz:
+                            return None
+                        some = np.zeros((x1 - x0 + 1, cells), dtype=bool)
+                        some.reshape(-1)[(x - x0) * cells + z // V] = True
+                        known[key] = int(np.count_nonzero(some, axis=1).max())
+                n = max(n, known[key])
+            most.append(n)
         return most
 
     def __init__(self, batch, plan, limits):
@@ -589,52 +605,68 @@ class ResidentTables(object):
         hc = -(-R // V)
         strips = plan.strips.copy()
         n = len(strips)
-        nz = np.array([s.shape[1] for s in batch.shots])
-        # nodes numbered over the shots, thus in strip order
-        base = np.cumsum([0] + [s.shape[0] * s.shape[1] for s in batch.shots])
+        # tables of the shots, made once for those that have the same entries
+        # and the same cut
+        known, ways, recs = {}, ([], []), []
 
-        def place(node):
-            """(strip, row in it, z) of nodes."""
-            si = np.searchsorted(base, node, side="right") - 1
-            x, z = np.divmod(node - base[si], nz[si])
-            st = plan.row_strip[plan.row_base[si] + x]
-            return st, x - strips[st, 1], z
+        def once(make, of, si, *more):
+            key = id(of), plan.cut_of[si], batch.shots[si].shape
+            if key not in known:
+                cut = plan.strips[plan.first_strip[si]:plan.first_strip[si + 1]]
+                known[key] = make(plan, cut, plan.row_strip[plan.cut_of[si]], batch.shots[si].shape[1], of, *more)
+            return known[key]
 
+        for si in range(batch.n_shots):
+            for way, nodes in enumerate((batch.src_nodes, batch.adj_nodes)):
+                ways[way].append(once(self._sources, nodes[si], si, V))
+            recs.append(once(self._receivers, batch.rec_nodes[si], si, batch.adj_nodes[si], R, hc, item))
         inj, fcells = [], np.zeros(n, dtype=np.int64)
-        for way, entries in enumerate(([s.src for s in batch.shots], [s.adj for s in batch.shots])):
-            si = np.repeat(np.arange(len(entries)), [e[0].shape[0] for e in entries])
-            pos, chan, w = (np.concatenate([e[i] for e in entries]) for i in range(3))
-            t = self._sources(plan, strips, place, base[si] + pos[:, 0] * nz[si] + pos[:, 1], chan, w, si, V, way)
-            fcells = np.maximum(fcells, t.pop("cells"))
-            inj.append(t)
+        for way, nodes in enumerate((batch.src_nodes, batch.adj_nodes)):
+            t = ways[way]
+            base = np.cumsum([0] + [ne.node.size for ne in nodes])
+            strips[:, 10 + 2 * way] = np.concatenate([b + x["first"][:-1] for b, x in zip(base, t)])
+            strips[:, 11 + 2 * way] = np.concatenate([b + x["first"][1:] for b, x in zip(base, t)])
+            fcells = np.maximum(fcells, np.concatenate([x["cells"] for x in t]))
+            # blocks of thread tables, one copy for alike shots
+            blocks, at, size = [], {}, 0
+            for x in t:
+                if id(x) not in at:
+                    at[id(x)] = size
+                    blocks.append(x["finfo"])
+                    size += len(x["finfo"])
+            strips[:, 29 + way] = np.concatenate([np.where(x["block"] < 0, -1, x["block"] + at[id(x)]) for x in t])
+            finfo = np.concatenate(blocks) if size else np.zeros((1, limits[2], 2), dtype=np.int32)
+            inj.append({"finfo": finfo, "lds": np.concatenate([x["lds"] for x in t])})
         strips[:, 24:28] = np.stack(lds_copies(strips, hc, R, fcells), axis=1)
         strips[:, 14:19] = lds_offsets(strips[:, 24:28].T, strips[:, 2], item).T
         # receiver nodes, in strip order
-        node = np.concatenate([b + idx for b, idx in zip(base, batch._rec_sorted)])
-        node, rec_node = _sorted_unique(node)
-        st, row, z = place(node)
-        rec_lds = (R + row) * (strips[st, 21] + hc) * 16 + hc * 16 + z * item
-        strips[:, 8] = np.searchsorted(st, np.arange(n))
-        strips[:, 9] = np.searchsorted(st, np.arange(n), side="right")
-        self.n_rec_nodes = node.size
+        base = np.cumsum([0] + [t["lds"].size for t in recs])
+        strips[:, 8] = np.concatenate([b + t["first"][:-1] for b, t in zip(base, recs)])
+        strips[:, 9] = np.concatenate([b + t["first"][1:] for b, t in zip(base, recs)])
+        rec_lds = np.concatenate([t["lds"] for t in recs])
+        rec_node = np.concatenate([t["node"] + np.int32(b) for b, t in zip(base, recs)])
+        self.n_rec_nodes = int(base[-1])
 
         # one upload, every table from a multiple of 16 bytes on
         tables = [strips, plan.items, rec_lds, rec_node]
         for t in inj:
-            tables += [t[k] for k in ("finfo", "lds", "nptr", "chan", "shot")]
+            tables += [t["finfo"], t["lds"]]
         at, size = [], 0
         for t in tables:
             at.append(size)
             size += -(-t.size // 4) * 4
-        weights = [np.ascontiguousarray(t["w"], dtype=np.float64).view(np.int32) for t in inj]
-        w_at = [size, size + weights[0].size]
         # (numpy: a tensor's fill wakes torch's threads, which then compete
         # with numpy's for milliseconds)
-        flat = np.zeros(size + weights[0].size + weights[1].size + 4, dtype=np.int32)
-        for a, t in zip(at + w_at, tables + weights):
+        flat = np.zeros(size + 4, dtype=np.int32)
+        for a, t in zip(at, tables):
             flat[a:a + t.size] = t.reshape(-1)
         self._tables = torch.from_numpy(flat).to(dev)
         ptr = self._tables.data_ptr()
+        # the nodes' entries {nptr, chan, w, shot}: the step kernels' tables
+        # where these have every shot's nodes in ascending order
+        self._entries = [inj[2:6] if by_node else self._node_entries(batch, nodes)
+                         for inj, by_node, nodes in ((batch.fwd_inj, batch.src_by_node, batch.src_nodes),
+                                                     (batch.adj_inj, batch.adj_by_node, batch.adj_nodes))]
         self.n_inj = [int(t["lds"].size) for t in inj]
         self.n_strips, self.cost = n, plan.cost
         self.group_begin = np.asarray(plan.group_begin, dtype=np.int32)
@@ -643,6 +675,8 @@ class ResidentTables(object):
         cells = 2 * -(-int(strips[:, 21].max()) // 64) * 64 * R
         stride = 2 * limits[4] * 4 + 4 * cells * 16
         self.xchg = torch.zeros(n * stride // 4, dtype=torch.int32, device=dev)
+        own = [t for way, by_node in zip(self._entries, (batch.src_by_node, batch.adj_by_node)) if not by_node for t in way]
+        self._fixed = sum(t.numel() * t.element_size() for t in [self._tables, self.xchg] + own)
         self.epoch = ctypes.c_uint(0)
         self._work, self._item = None, item
         self._slot_bytes = (max(1, max(self.n_inj)) + max(1, self.n_rec_nodes)) * item
@@ -652,9 +686,8 @@ class ResidentTables(object):
         q.group_lds = self.group_lds.ctypes.data
         q.strips, q.items, q.rec_lds, q.rec_node = (ptr + 4 * a for a in at[:4])
         for way in range(2):
-            (q.finfo[way], q.inj_lds[way], q.inj_nptr[way], q.inj_chan[way],
-             q.inj_shot[way]) = (ptr + 4 * a for a in at[4 + 5 * way:9 + 5 * way])
-            q.inj_w[way] = ptr + 4 * w_at[way]
+            q.finfo[way], q.inj_lds[way] = (ptr + 4 * a for a in at[4 + 2 * way:6 + 2 * way])
+            q.inj_nptr[way], q.inj_chan[way], q.inj_w[way], q.inj_shot[way] = (t.data_ptr() for t in self._entries[way])
             q.n_inj[way] = self.n_inj[way]
         q.n_rec_nodes = self.n_rec_nodes
         q.xchg, q.xchg_stride, q.xchg_cells = self.xchg.data_ptr(), stride, cells
@@ -666,37 +699,58 @@ class ResidentTables(object):
         q.epoch = ctypes.addressof(self.epoch)
 
     @staticmethod
-    def _sources(plan, strips, place, pos, chan, w, shot, V, way):
-        """Source tables in strip order: nodes, each with its entries in the
-        given order; for the strips with sources, per thread the first source
-        cell and the march steps that have one (a block of ``finfo``, which
-        the strip's number 29 + way names); source cells of every strip."""
+    def _node_entries(batch, nodes):
+        """Device arrays {nptr, chan, w, shot} of the nodes' entries."""
+        base = np.cumsum([0] + [ne.chan.size for ne in nodes])
+        nptr = np.concatenate([b + ne.nptr[:-1] for b, ne in zip(base, nodes)] + [base[-1:]])
+        shot = np.repeat(np.arange(len(nodes)), [ne.node.size for ne in nodes])
+        return batch._send([(np.int32, [nptr]), (np.int32, [ne.chan for ne in nodes]),
+                            (np.float64, [ne.w for ne in nodes]), (np.int32, [shot])])
+
+    @staticmethod
+    def _sources(plan, strips, row_strip, nz, nodes, V):
+        """Source tables of one shot with these ``strips``: where a node's
+        value lies among its strip's source cells (``lds``); per strip the
+        first of its nodes and its source cells; for the strips with sources
+        (``block``: their number, or -1), per thread the first source cell and
+        the march steps that have one (``finfo``)."""
         n, threads = len(strips), plan.items.shape[1]
-        if pos.size and np.any(pos[1:] < pos[:-1]):
-            order = np.argsort(pos, kind="stable")
-            pos, chan, w, shot = (a[order] for a in (pos, chan, w, shot))
-        first = np.nonzero(np.concatenate([[True], pos[1:] != pos[:-1]]))[0] if pos.size else np.zeros(0, dtype=np.int64)
-        st, row, z = place(pos[first])
-        strips[:, 10 + 2 * way] = np.searchsorted(st, np.arange(n))
-        strips[:, 11 + 2 * way] = np.searchsorted(st, np.arange(n), side="right")
+        x, z = np.divmod(nodes.node, nz)
+        st = row_strip[x]
+        row = x - strips[st, 1]
         own = plan.owner[plan.owner_base[strips[st, 28]] + row * strips[st, 21] + z // V]
         # a strip's cells in the order its threads march over them
         key = (st * threads + own[:, 0]) * 64 + own[:, 1]
         cells, inv = np.unique(key, return_inverse=True)
         owner, step = cells // 64, cells % 64
         begin = np.searchsorted(owner // threads, np.arange(n + 1))
-        lds = (inv.reshape(-1) - begin[st]) * V + z % V
         some = np.nonzero(begin[1:] > begin[:-1])[0]
-        strips[:, 29 + way] = -1
-        strips[some, 29 + way] = np.arange(some.size)
-        finfo = np.zeros((max(1, some.size), threads, 2), dtype=np.int32)
+        block = np.full(n, -1)
+        block[some] = np.arange(some.size)
+        finfo = np.zeros((some.size, threads, 2), dtype=np.int32)
         if some.size:
             heads = np.nonzero(np.concatenate([[True], owner[1:] != owner[:-1]]))[0]
             k, t = np.divmod(owner[heads], threads)
-            finfo[strips[k, 29 + way], t, 0] = heads - begin[k]
-            finfo[strips[k, 29 + way], t, 1] = np.bitwise_or.reduceat(1 << step, heads)
-        return {"lds": lds, "nptr": np.append(first, pos.size), "chan": chan, "w": w, "shot": shot[first],
-                "finfo": finfo, "cells": np.diff(begin)}
+            finfo[block[k], t, 0] = heads - begin[k]
+            finfo[block[k], t, 1] = np.bitwise_or.reduceat(1 << step, heads)
+        return {"lds": (inv.reshape(-1) - begin[st]) * V + z % V, "first": np.searchsorted(st, np.arange(n + 1)),
+                "finfo": finfo, "block": block, "cells": np.diff(begin)}
+
+    @staticmethod
+    def _receivers(plan, strips, row_strip, nz, rec, adj, R, hc, item):
+        """Receiver tables of one shot with these ``strips``: where a node
+        lies in LDS, the first node of every strip, and the node of every
+        entry (flat nodes ``rec``, in most batches those of the adjoint
+        entries ``adj``)."""
+        if np.array_equal(rec, adj.given):
+            node, of = adj.node, adj.rank()
+        else:
+            node, of = np.unique(rec, return_inverse=True)
+            of = of.reshape(-1).astype(np.int32)
+        x, z = np.divmod(node, nz)
+        st = row_strip[x]
+        lds = (R + x - strips[st, 1]) * (strips[st, 21] + hc) * 16 + hc * 16 + z * item
+        return {"lds": lds, "first": np.searchsorted(st, np.arange(len(strips) + 1)), "node": of}
 
     def chunk_slots(self, max_nt, budget):
         """Slots of a run of ``max_nt`` that are worked on at a time: what
@@ -713,12 +767,11 @@ class ResidentTables(object):
         runs of up to ``max_nt`` slots: tables, border rows, working space,
         and the sources of a run too short for the loop."""
         short = max(self.n_inj) * min(max_nt, RESIDENT_MIN_SLOTS - 1) * self._item
-        return (self._tables.numel() + self.xchg.numel()) * 4 + self._slot_bytes * self.chunk_slots(max_nt, budget) \
-            + short
+        return self._fixed + self._slot_bytes * self.chunk_slots(max_nt, budget) + short
 
     def held(self):
         """Bytes of what ``reserve`` counts that are allocated."""
-        return (self._tables.numel() + self.xchg.numel()) * 4 + (self._work[0] * self._slot_bytes if self._work else 0)
+        return self._fixed + (self._work[0] * self._slot_bytes if self._work else 0)
 
     def _workspace(self, batch):
         """Source values and receiver nodes of a chunk of slots."""

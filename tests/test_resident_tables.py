@@ -239,3 +239,119 @@ def test_a_kept_plan_belongs_to_its_grouping(monkeypatch):
     monkeypatch.setattr(resident, "plan_groups", lambda shots, cus: rule(shots, len(shots[0].cut(1e9))))
     other = resident.Plan.of(keys, 4, 8, LIMITS, 256)
     assert len(one.group_begin) == 2 and len(other.group_begin) > 2
+
+
+def _on_cpu(monkeypatch):
+    """Batches whose tables are built in host memory."""
+    import torch
+    from pysit_amd import device
+    monkeypatch.setattr(resident.N, "resident_limits", lambda: LIMITS)
+    monkeypatch.setattr(resident.N, "tile_rows", lambda dim, code, axis: (16, 8)[axis] if dim == 3 else 8)
+    monkeypatch.setattr(device, "_dev", lambda: torch.device("cpu"))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda dev: _Device)
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda self, *a: self)
+    return device.DeviceBatch
+
+
+def _shared(probs, seed):
+    """Geometries of which the odd ones share the first one's receivers, given
+    in no order, as a survey's shots share an operator."""
+    g = [p.geometry() for p in probs]
+    order = np.random.default_rng(seed).permutation(g[0].adj[1].size)
+    g[0].adj = tuple(a[order] for a in g[0].adj)
+    g[0].rec = tuple(a[order[::-1]] for a in g[0].rec)
+    for other in g[1::2]:
+        other.adj, other.rec, other.nrec = g[0].adj, g[0].rec, g[0].nrec
+    return g
+
+
+@pytest.mark.parametrize("shape,tiles", [((70, 150), "shot"), ((70, 150), "interleave"), ((20, 30, 140), "shot")])
+def test_entry_tables_hold_every_entry_in_its_order(monkeypatch, shape, tiles):
+    """The injection and receiver tables against the entries one by one:
+    tiles, then nodes, then the entries of a node as given; receivers' entries
+    as given; also where shots share their entries."""
+    from tests.problems import Synthetic
+    make = _on_cpu(monkeypatch)
+    dim = len(shape)
+    probs = [Synthetic(shape, ((4, 5),) * dim, (0.01,) * dim, 12, 4, seed=i, n_rec=9, n_src=2) for i in range(3)]
+    b = make(_shared(probs, 1), probs[0].model, (0.01,) * dim, probs[0].dt, 4, tile_order=tiles)
+    lists = {tuple(t[:2]): i for i, t in enumerate(b.tiles.numpy().reshape(-1, 4))}
+    for tables, entries in ((b.fwd_inj, [s.src for s in b.shots]), (b.adj_inj, [s.adj for s in b.shots])):
+        want = {}
+        for si, (pos, chan, w) in enumerate(entries):
+            tile, local = b._tile_of_pos(b.shots[si], b.tiles_info[si][0], pos)
+            for t, l, c, v in zip(tile, local, chan, w):
+                want.setdefault((lists[si, t], int(l)), []).append((si, c, v))
+        ptr, node, nptr, chan, w, shot = (t.numpy() for t in tables)
+        got = {}
+        for t in range(b.n_tiles):
+            for n in range(ptr[t], ptr[t + 1]):
+                got[t, int(node[n])] = [(shot[n], chan[e], w[e]) for e in range(nptr[n], nptr[n + 1])]
+        assert list(got) == sorted(want) and got == want
+    recs, at, w = b.recs.numpy().reshape(-1, 4), b.rec_idx.numpy(), b.rec_w.numpy()
+    rows = iter(recs)
+    for si, s in enumerate(b.shots):
+        idx = (s.rec[0] // shape[-1]) * b.zs[si] + s.rec[0] % shape[-1]
+        for r in range(s.nrec):
+            shot, k, e0, e1 = next(rows)
+            mine = s.rec[1] == r
+            assert (shot, k) == (si, r) and np.array_equal(at[e0:e1], idx[mine]) and np.array_equal(w[e0:e1], s.rec[2][mine])
+
+
+@pytest.mark.parametrize("z", [30, 63])
+def test_resident_entries_of_shared_operators(monkeypatch, z):
+    """The loop's source and receiver tables against the entries one by one,
+    where shots share entries and have their nodes in one z tile or in two."""
+    import ctypes
+    from tests.problems import Synthetic
+    make = _on_cpu(monkeypatch)
+    probs = [Synthetic((150, 130), ((6, 7), (5, 8)), (0.01, 0.01), 12, 8, seed=i, n_rec=9, rec_z=z) for i in range(3)]
+    b = make(_shared(probs, 2), probs[0].model, (0.01, 0.01), probs[0].dt, 8, resident=True)
+    assert b.adj_by_node == (z == 30)
+    q, R, V, hc = b.resident_tables().struct, 4, 4, 1
+
+    def view(ptr, n, kind=ctypes.c_int):
+        return np.ctypeslib.as_array(ctypes.cast(ptr, ctypes.POINTER(kind)), (n,))
+
+    strips = view(q.strips, 32 * q.n_strips).reshape(-1, 32)
+    plan = resident.ResidentTables.plan(b.shots, R, 4, b.dev, True)
+
+    def strip_of(si, node):
+        x, zz = divmod(int(node), b.shots[si].shape[1])
+        st = [k for k, d in enumerate(strips) if d[0] == si and d[1] <= x < d[1] + d[2]]
+        assert len(st) == 1
+        return st[0], x - int(strips[st[0]][1]), zz
+
+    for way, entries in enumerate(([s.src for s in b.shots], [s.adj for s in b.shots])):
+        n = q.n_inj[way]
+        nptr = view(q.inj_nptr[way], n + 1)
+        chan, w = view(q.inj_chan[way], nptr[-1]), view(q.inj_w[way], nptr[-1], ctypes.c_double)
+        lds, shot = view(q.inj_lds[way], n), view(q.inj_shot[way], n)
+        finfo = view(q.finfo[way], 1024 * (1 + strips[:, 29 + way].max())).reshape(-1, 512, 2)
+        i = 0
+        for si, (pos, c, v) in enumerate(entries):
+            flat = pos[:, 0] * 130 + pos[:, 1]
+            for node in np.unique(flat):
+                mine = flat == node
+                assert shot[i] == si and np.array_equal(chan[nptr[i]:nptr[i + 1]], c[mine])
+                assert np.array_equal(w[nptr[i]:nptr[i + 1]], v[mine])
+                st, row, zz = strip_of(si, node)
+                d = strips[st]
+                assert d[10 + 2 * way] <= i < d[11 + 2 * way]
+                # the thread that owns the cell reads it where the value is put
+                t, step = plan.owner[plan.owner_base[d[28]] + row * d[21] + zz // V]
+                first, steps = finfo[d[29 + way], t]
+                assert steps >> step & 1
+                assert lds[i] == (first + bin(steps & ((1 << step) - 1)).count("1")) * V + zz % V
+                i += 1
+        assert i == n
+    lds, at = view(q.rec_lds, q.n_rec_nodes), view(q.rec_node, len(b.rec_w))
+    e = 0
+    for si, s in enumerate(b.shots):
+        for node in s.rec[0][np.argsort(s.rec[1], kind="stable")]:
+            st, row, zz = strip_of(si, node)
+            d = strips[st]
+            assert d[8] <= at[e] < d[9] and lds[at[e]] == ((R + row) * (d[21] + hc) + hc) * 16 + zz * 4
+            e += 1
+    assert e == len(b.rec_w)
