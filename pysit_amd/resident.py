@@ -46,6 +46,9 @@ STEP_KERNEL_BYTES = 30000.0
 # such a batch 1 %
 CHUNK_BYTES = 256 << 20
 CHUNK_SHARE = 16
+# slots of a chunk at most: the receivers' kernel takes 8 slots a workgroup
+# along its grid's second axis, which has 65535 at most
+CHUNK_SLOTS = 8 * 65535
 # shorter runs than this many slots go through the step kernels: a resident
 # launch loads and stores the whole state
 RESIDENT_MIN_SLOTS = 8
@@ -760,7 +763,7 @@ class ResidentTables(object):
         room, least = CHUNK_BYTES, 32
         if budget is not None:
             room, least = min(CHUNK_BYTES, int(budget) // CHUNK_SHARE), RESIDENT_MIN_SLOTS
-        return min(max_nt, max(least, room // self._slot_bytes))
+        return min(max_nt, max(least, min(CHUNK_SLOTS, room // self._slot_bytes)))
 
     def reserve(self, max_nt, budget):
         """Bytes that the loop takes beside the batch's state and stores in

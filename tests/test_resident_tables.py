@@ -355,3 +355,16 @@ def test_resident_entries_of_shared_operators(monkeypatch, z):
             assert d[8] <= at[e] < d[9] and lds[at[e]] == ((R + row) * (d[21] + hc) + hc) * 16 + zz * 4
             e += 1
     assert e == len(b.rec_w)
+
+
+def test_chunks_of_a_long_run_fit_the_grid():
+    """A record of few receivers and many steps is cut to chunks that the
+    receivers' kernel can number."""
+    t = object.__new__(resident.ResidentTables)
+    for nodes in (1, 10, 84, 100000):
+        t._slot_bytes = nodes * 4
+        for nt in (5, 100, 10 ** 6, 10 ** 8):
+            for budget in (None, 10 ** 6, 10 ** 11):
+                slots = t.chunk_slots(nt, budget)
+                assert 1 <= slots <= nt and -(-slots // 8) <= 65535
+                assert slots * t._slot_bytes <= max(resident.CHUNK_BYTES, 32 * t._slot_bytes)
