@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from . import _native as N
-from .resident import RESIDENT_MIN_SLOTS, ResidentTables
+from .resident import CHUNK_BYTES, RESIDENT_MIN_SLOTS, ResidentTables
 
 TILE_Z = 64      # z nodes per wavefront (the contiguous axis)
 
@@ -1000,6 +1000,8 @@ class DeviceBatch:
         batch goes on with the step kernels."""
         self.snaps = None
         if not keep_dw:
+            if self.memory_budget is not None and self.dw is None and self.resident_tables():
+                self.resident_tables().room = self.memory_budget // 2
             return self.max_nt
         if self.schedule not in ("auto", "binomial"):
             raise ValueError("schedule must be 'auto' or 'binomial'")
@@ -1022,7 +1024,9 @@ class DeviceBatch:
 
     def _plan_budget(self, tables):
         """``plan_segments`` with the buffers of the resident loop's
-        ``tables`` counted, or without the loop."""
+        ``tables`` counted, or without the loop.  Under a budget the loop's
+        working space is the least it runs with; what the schedule leaves over
+        goes to it as well (``tables.room``)."""
         self.snaps = None
         budget = self.memory_budget
         item = self.dtype.itemsize
@@ -1030,7 +1034,7 @@ class DeviceBatch:
         per_slot = (self.total_n + n_inj) * item
         ckpt = self.ckpt_bytes()
         state = self.state_bytes()
-        loop = tables.reserve(self.max_nt, budget) if tables else 0
+        loop = tables.reserve(self.max_nt, CHUNK_BYTES if budget is None else 0) if tables else 0
         if budget is None:
             # everything this batch holds from an earlier gradient counts as
             # available (a new one reuses or releases it), so repeated calls
@@ -1053,12 +1057,23 @@ class DeviceBatch:
         if self.schedule == "binomial":
             return self._plan_binomial(budget, per_slot, ckpt, state)
         if self.max_nt * per_slot <= budget:
+            if tables:
+                tables.room = budget - self.max_nt * self.total_n * item
             return self.max_nt
+        if tables and (self.dtype == np.float64 or self.ic_window):
+            # the adjoint's sources are in the loop's working space
+            per_slot = self.total_n * item
         levels = checkpoint_levels(self.max_nt, per_slot, ckpt, budget, state=state)
         if levels is None:
             # fewer bytes than the nested schedule needs: state snapshots
             # alone, reversed step by step (binomial schedule)
             return self._plan_binomial(budget, per_slot, ckpt, state)
+        if tables and self.memory_budget is not None:
+            if len(levels) == 1:
+                # the segments' number is what costs: equal ones leave more room
+                levels = [-(-self.max_nt // -(-self.max_nt // levels[0]))]
+            counts = [-(-a // k) for a, k in zip([self.max_nt] + levels, levels)]
+            tables.room = budget - levels[-1] * per_slot - sum(counts) * ckpt - state
         held = getattr(self, "dw_slots", 0) if getattr(self, "dw", None) is not None else 0
         if (self.memory_budget is None and len(levels) == 1 and held and held == getattr(self, "K", 0)
                 and abs(levels[0] - held) <= max(2, levels[0] // 20)):
@@ -1075,6 +1090,8 @@ class DeviceBatch:
         adjoint reverses the run from rest with as many state snapshots as
         fit (a working state and a one-slot dWaveOp store beside them), each
         reverse step recomputing its own dWaveOp.  Returns K = 1."""
+        if self._resident:
+            self._resident.room = 0
         snaps = (budget - state - per_slot) // ckpt
         if snaps < 0:
             raise MemoryError("memory budget too small for the checkpoint schedule")
@@ -1121,6 +1138,8 @@ class DeviceBatch:
         if segment:
             K = int(segment)
             self.levels = [K]
+            if self.resident_tables():
+                self.resident_tables().room = K * self.resident_tables().slot_bytes
         else:
             K = self.plan_segments(keep_dw)
         self.K = K
@@ -1496,6 +1515,8 @@ class DeviceBatch:
             return
         if not self._resident:
             slots = b.sweep_slots
+        elif slots >= RESIDENT_MIN_SLOTS and self.memory_budget is not None:
+            self._resident.release()  # a schedule counts the larger of the two
         b.inj_pre = self._inj_pre_buffer(slots, n_nodes).data_ptr()
         b.inj_node_shot = self.adj_inj[5].data_ptr()
         b.n_inj_nodes = n_nodes

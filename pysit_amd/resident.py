@@ -40,12 +40,13 @@ SHARE_COST = 1.0
 # and the bytes of one field that add 1
 STEP_KERNEL_COST = 35.0
 STEP_KERNEL_BYTES = 30000.0
-# device memory for the source values and receiver nodes of a chunk of slots,
-# and its part of a memory budget that a caller sets: 1/16 of 4 GB holds 700
-# slots of 16 shots of 1041 x 341 nodes, and a launch more per 100 slots costs
-# such a batch 1 %
+# device memory for the source values and receiver nodes of a chunk of slots
+# where no memory budget is set, and the slots a chunk has at least: each chunk
+# is a launch, which loads and stores the state (55 us for 1 shot of
+# 1041 x 341 nodes or 4 of 541 x 241, 100 us for 16 of 1041 x 341; a step takes
+# 6, 7 and 18 us)
 CHUNK_BYTES = 256 << 20
-CHUNK_SHARE = 16
+CHUNK_LEAST = 32
 # slots of a chunk at most: the receivers' kernel takes 8 slots a workgroup
 # along its grid's second axis, which has 65535 at most
 CHUNK_SLOTS = 8 * 65535
@@ -682,7 +683,9 @@ class ResidentTables(object):
         self._fixed = sum(t.numel() * t.element_size() for t in [self._tables, self.xchg] + own)
         self.epoch = ctypes.c_uint(0)
         self._work, self._item = None, item
-        self._slot_bytes = (max(1, max(self.n_inj)) + max(1, self.n_rec_nodes)) * item
+        self.slot_bytes = max(1, self.n_inj[0] + self.n_rec_nodes, self.n_inj[1]) * item
+        # bytes of working space under a memory budget (DeviceBatch.plan_segments)
+        self.room = 0
         q = self.struct = N.Resident()
         q.n_strips, q.n_groups = n, len(self.group_lds)
         q.group_begin = self.group_begin.ctypes.data
@@ -755,41 +758,44 @@ class ResidentTables(object):
         lds = (R + x - strips[st, 1]) * (strips[st, 21] + hc) * 16 + hc * 16 + z * item
         return {"lds": lds, "first": np.searchsorted(st, np.arange(len(strips) + 1)), "node": of}
 
-    def chunk_slots(self, max_nt, budget):
+    def chunk_slots(self, max_nt, room):
         """Slots of a run of ``max_nt`` that are worked on at a time: what
-        CHUNK_BYTES, or the working space's share of a memory ``budget`` if
-        there is one, hold of source values and receiver nodes, and 32 or 8
-        at least."""
-        room, least = CHUNK_BYTES, 32
-        if budget is not None:
-            room, least = min(CHUNK_BYTES, int(budget) // CHUNK_SHARE), RESIDENT_MIN_SLOTS
-        return min(max_nt, max(least, min(CHUNK_SLOTS, room // self._slot_bytes)))
+        ``room`` bytes hold of source values and receiver nodes, or
+        CHUNK_LEAST."""
+        return min(max_nt, max(CHUNK_LEAST, min(CHUNK_SLOTS, room // self.slot_bytes)))
 
-    def reserve(self, max_nt, budget):
+    def reserve(self, max_nt, room):
         """Bytes that the loop takes beside the batch's state and stores in
-        runs of up to ``max_nt`` slots: tables, border rows, working space,
-        and the sources of a run too short for the loop."""
-        short = max(self.n_inj) * min(max_nt, RESIDENT_MIN_SLOTS - 1) * self._item
-        return self._fixed + self._slot_bytes * self.chunk_slots(max_nt, budget) + short
+        runs of up to ``max_nt`` slots: tables, border rows, working space in
+        ``room`` bytes, and the sources of a run too short for the loop."""
+        short = self.n_inj[1] * min(max_nt, RESIDENT_MIN_SLOTS - 1) * self._item
+        return self._fixed + self.slot_bytes * self.chunk_slots(max_nt, room) + short
 
     def held(self):
         """Bytes of what ``reserve`` counts that are allocated."""
-        return self._fixed + (self._work[0] * self._slot_bytes if self._work else 0)
+        return self._fixed + (self._work[0] * self.slot_bytes if self._work else 0)
+
+    def release(self):
+        """Give the working space back; the next run takes it again."""
+        self._work = None
 
     def _workspace(self, batch):
-        """Source values and receiver nodes of a chunk of slots."""
+        """Source values and receiver nodes of a chunk of slots, one behind
+        the other: a forward run has few sources, an adjoint no receivers."""
         import torch
-        slots = self.chunk_slots(batch.max_nt, batch.memory_budget)
+        slots = self.chunk_slots(batch.max_nt, CHUNK_BYTES if batch.memory_budget is None else min(CHUNK_BYTES, self.room))
         have = self._work[0] if self._work else 0
         # a larger one stays where nothing bounds it (the time axis may change again)
         if have < slots or (have > slots and batch.memory_budget is not None):
-            self._work = None  # first: both together may not fit
-            pre = torch.empty(slots * max(1, max(self.n_inj)), dtype=batch.tdtype, device=batch.dev)
-            rec = torch.empty(slots * max(1, self.n_rec_nodes), dtype=batch.tdtype, device=batch.dev)
-            self._work = (slots, pre, rec)
-            q = self.struct
-            q.pre, q.recbuf = pre.data_ptr(), rec.data_ptr()
-            q.pre_slots = q.rec_slots = slots
+            self._work = None  # first: both together may not fit, nor this and a long run's sources for the step kernels
+            if batch.memory_budget is not None:
+                batch._inj_pre = None
+            self._work = slots, torch.empty(slots * self.slot_bytes // self._item, dtype=batch.tdtype, device=batch.dev)
+        slots, work = self._work
+        q = self.struct
+        q.pre_slots = q.rec_slots = slots
+        q.pre = work.data_ptr()
+        q.recbuf = work.data_ptr() + slots * self.n_inj[0] * self._item
 
     def expired(self):
         """Whether a wait for a neighbour ran into its bound in a run that the

@@ -181,13 +181,14 @@ def test_a_batch_is_built_once_whichever_loop_takes_it(monkeypatch, shape, pml, 
 
 
 class _Loop(object):
-    """Resident tables that take ``size`` bytes."""
+    """Resident tables that take ``size`` bytes and ``slot`` bytes of working
+    space per slot, 32 slots at least."""
 
-    def __init__(self, size):
-        self.size = size
+    def __init__(self, size, slot):
+        self.size, self.slot_bytes, self.room = size, slot, 0
 
-    def reserve(self, max_nt, budget):
-        return self.size
+    def reserve(self, max_nt, room):
+        return self.size + self.slot_bytes * max(32, room // self.slot_bytes)
 
     def held(self):
         return 0
@@ -196,38 +197,42 @@ class _Loop(object):
 @pytest.mark.parametrize("loop", [0, 1000, 40000, 10 ** 9])
 def test_a_memory_budget_counts_the_loop(loop):
     """The schedule leaves room for the loop's buffers; where they would cost
-    a level of the schedule's kind or all of it, the batch does without them,
-    and a budget that held a schedule before still does."""
+    the kind of the schedule or all of it, the batch does without them, and a
+    budget that held a schedule before still does.  What is left over goes to
+    the working space, and segments stay as few as the budget holds."""
     import torch
     from pysit_amd import device
     nt, n, nodes = 200, 1000, 30
 
     def batch(budget, tables):
         b = object.__new__(device.DeviceBatch)
-        b._resident, b.schedule, b.memory_budget, b.max_snaps = tables, "auto", budget, None
-        b.dtype, b.dim, b.total_n, b.max_nt = np.dtype(np.float32), 2, n, nt
+        b._resident, b.schedule, b.memory_budget, b.max_snaps, b.ic_window = tables, "auto", budget, None, 64
+        b.dtype, b.dim, b.total_n, b.max_nt, b.dw = np.dtype(np.float32), 2, n, nt, None
         b.adj_inj = (None, None, torch.zeros(nodes + 1))
         return b
 
-    state, ckpt, slot = 7 * n * 4, 4 * n * 4, (n + nodes) * 4
-    for budget in range(state + 12 * n + 60000, state + 12 * n + nt * slot + 20000, 7777):
+    state, ckpt, slot, base = 7 * n * 4, 4 * n * 4, n * 4, 7 * n * 4 + 12 * n
+    for budget in range(base + 60000, base + nt * (slot + nodes * 4) + 40000, 7777):
         plain = batch(budget, False)
         try:
             K = plain.plan_segments(True)
         except MemoryError:
             continue
-        b = batch(budget, _Loop(loop))
+        b = batch(budget, _Loop(loop, 2 * nodes * 4))
         Kb = b.plan_segments(True)
-        size = loop if b._resident else 0
         assert (plain.snaps is None) == (b.snaps is None)
-        if b.snaps is None:
+        if b._resident is False:
+            assert Kb == K and b.levels == plain.levels
+        elif b.snaps is None:
+            t = b._resident
             levels = b.levels if Kb < nt else []
             counts = [-(-a // k) for a, k in zip([nt] + levels, levels)]
-            stored = (levels or [nt])[-1]
-            need = stored * slot + sum(counts) * ckpt + (state if levels else 0)
-            assert need + size + state + 12 * n <= budget
-            if not b._resident:
-                assert Kb == K and b.levels == plain.levels and loop > 0
+            need = (levels or [nt])[-1] * slot + sum(counts) * ckpt + (state if levels else 0)
+            work = max(t.room, 32 * t.slot_bytes)
+            assert t.room >= 0 and base + need + loop + work <= budget
+            if len(levels) == 1:  # one segment fewer would not fit
+                fewer = counts[0] - 1
+                assert fewer == 0 or base + -(-nt // fewer) * slot + fewer * ckpt + state + loop + 32 * t.slot_bytes > budget
 
 
 def test_a_kept_plan_belongs_to_its_grouping(monkeypatch):
@@ -362,9 +367,9 @@ def test_chunks_of_a_long_run_fit_the_grid():
     receivers' kernel can number."""
     t = object.__new__(resident.ResidentTables)
     for nodes in (1, 10, 84, 100000):
-        t._slot_bytes = nodes * 4
+        t.slot_bytes = nodes * 4
         for nt in (5, 100, 10 ** 6, 10 ** 8):
-            for budget in (None, 10 ** 6, 10 ** 11):
-                slots = t.chunk_slots(nt, budget)
+            for room in (0, 10 ** 6, resident.CHUNK_BYTES, 10 ** 11):
+                slots = t.chunk_slots(nt, room)
                 assert 1 <= slots <= nt and -(-slots // 8) <= 65535
-                assert slots * t._slot_bytes <= max(resident.CHUNK_BYTES, 32 * t._slot_bytes)
+                assert slots * t.slot_bytes <= max(room, 32 * t.slot_bytes)
