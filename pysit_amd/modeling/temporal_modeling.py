@@ -173,14 +173,22 @@ class TemporalModeling(object):
         return DeviceBatch(geometries, model, s.mesh.deltas, s.dt, s.spatial_accuracy_order, tile_x=self.tile_x,
                            **kw)
 
-    def _host(self, batch, t):
-        """Result tensor ``t`` of ``batch`` on the host, checked."""
-        a = t.cpu().numpy()
+    def check(self, batch=None):
+        """Raise if a wait of the resident loop expired in a run of ``batch``
+        (default: the one kept for reuse) that the host has waited for."""
+        if batch is None:
+            batch = getattr(self, "_batch_cache", None) and self._batch_cache[1]
         try:
-            batch.check()
+            if batch is not None:
+                batch.check()
         except NativeError:
             self._step_kernels = True
             raise
+
+    def _host(self, batch, t):
+        """Result tensor ``t`` of ``batch`` on the host, checked."""
+        a = t.cpu().numpy()
+        self.check(batch)
         return a
 
     def _unpad_field(self, padded):

@@ -150,6 +150,7 @@ class TemporalLeastSquares(object):
                 s2 = torch.sum(r * r)
                 r2 = s2 if r2 is None else r2 + s2
         r2 = float(self._allreduce(np.array(0.0 if r2 is None else float(r2))))
+        self.modeling_tools.check()
         return 0.5 * r2 * self.solver.dt
 
     def _gradient_helper(self, shot, m0, ignore_minus=False, **kwargs):

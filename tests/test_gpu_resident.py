@@ -222,3 +222,22 @@ def test_short_adjoint_segments_precompute_their_sources(gpu):
     out = _gradient(held, _residuals([p]), segment=30)
     assert _same(out[0], ref[0]) and _same(out[1], ref[1])
     assert held._inj_pre.numel() == 7 * (held.adj_inj[2].numel() - 1)  # slots 90 to 96
+
+
+def test_evaluate_raises_for_an_expired_wait(gpu, monkeypatch):
+    """The objective alone, whose traces never reach the host."""
+    import pysit_amd as pa
+    from pysit_amd import _native as N
+    from pysit_amd import resident
+    from tests.problems import c1_setup
+    m, shots, solver, model = c1_setup(tf=0.3)
+    pa.generate_seismic_data(shots, solver, model)
+    trial = solver.ModelParameters(m, {"C": 1.01 * model.C})
+    want = pa.TemporalLeastSquares(solver).evaluate(shots, trial)
+    assert np.isfinite(want) and want > 0
+    monkeypatch.setattr(resident, "SPIN", 1)
+    obj = pa.TemporalLeastSquares(solver)
+    print("resident expired evaluate", flush=True)
+    with pytest.raises(N.NativeError, match="waited too long"):
+        obj.evaluate(shots, trial)
+    assert obj.evaluate(shots, trial) == want
