@@ -1171,7 +1171,7 @@ class DeviceBatch:
                 # as available: release it before the checkpoints are taken
                 self.dw = None
                 self.dw_slots = 0
-                self._inj_pre = None
+                self.release_sources()
                 torch.cuda.empty_cache()
             b = self._batch(self.fstate, False)
             one_level = len(getattr(self, "levels", [K])) == 1
@@ -1522,13 +1522,20 @@ class DeviceBatch:
         b.n_inj_nodes = n_nodes
         b.inj_pre_slots = slots
 
+    def release_sources(self):
+        """Give the precomputed sources back once the current stream is done
+        with them (their own stream may be another)."""
+        if getattr(self, "_inj_pre", None) is not None:
+            self._inj_pre.record_stream(torch.cuda.current_stream())
+        self._inj_pre = None
+
     def _inj_pre_buffer(self, slots, n_nodes):
         """Device buffer for the precomputed injection of ``slots`` slots
         (kept between calls)."""
         need = slots * n_nodes
         buf = getattr(self, "_inj_pre", None)
         if buf is None or buf.numel() < need:
-            self._inj_pre = None
+            self.release_sources()
             buf = self._inj_pre = torch.empty(need, dtype=self.tdtype, device=self.dev)
         return buf
 

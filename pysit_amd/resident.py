@@ -776,7 +776,11 @@ class ResidentTables(object):
         return self._fixed + (self._work[0] * self.slot_bytes if self._work else 0)
 
     def release(self):
-        """Give the working space back; the next run takes it again."""
+        """Give the working space back once the current stream is done with
+        it (its own stream may be another); the next run takes it again."""
+        import torch
+        if self._work is not None:
+            self._work[1].record_stream(torch.cuda.current_stream())
         self._work = None
 
     def _workspace(self, batch):
@@ -787,9 +791,10 @@ class ResidentTables(object):
         have = self._work[0] if self._work else 0
         # a larger one stays where nothing bounds it (the time axis may change again)
         if have < slots or (have > slots and batch.memory_budget is not None):
-            self._work = None  # first: both together may not fit, nor this and a long run's sources for the step kernels
+            # first: both together may not fit, nor this and a long run's sources for the step kernels
+            self.release()
             if batch.memory_budget is not None:
-                batch._inj_pre = None
+                batch.release_sources()
             self._work = slots, torch.empty(slots * self.slot_bytes // self._item, dtype=batch.tdtype, device=batch.dev)
         slots, work = self._work
         q = self.struct

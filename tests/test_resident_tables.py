@@ -373,3 +373,28 @@ def test_chunks_of_a_long_run_fit_the_grid():
                 slots = t.chunk_slots(nt, room)
                 assert 1 <= slots <= nt and -(-slots // 8) <= 65535
                 assert slots * t.slot_bytes <= max(room, 32 * t.slot_bytes)
+
+
+def test_buffers_given_back_wait_for_the_stream_that_used_them(monkeypatch):
+    """A working space or source buffer dropped by a run on another stream
+    than it was allocated on is not given out before that run is done."""
+    import torch
+    from pysit_amd import device
+    used = []
+
+    class Buffer(object):
+        def record_stream(self, stream):
+            used.append((self, stream))
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: "other")
+    t = object.__new__(resident.ResidentTables)
+    work = Buffer()
+    t._work = 32, work
+    t.release()
+    assert t._work is None and used == [(work, "other")]
+    t.release()
+    b = object.__new__(device.DeviceBatch)
+    b.release_sources()
+    b._inj_pre = Buffer()
+    b.release_sources()
+    assert b._inj_pre is None and len(used) == 2
