@@ -364,8 +364,8 @@ def run_c1(args):
                    "nt": nt, "grid_padded": list(shape)},
         "vs_oracle": {"traces_rel_l2": rel(sim, ref["simdata"]), "gradient_rel_l2": rel(g.data, grad_ref)},
         "residency": f"the state ({7 * n * 8 / 2**20:.1f} MiB of FP64 fields) and the dWaveOp history "
-                     f"({nt * n * 8 / 2**20:.0f} MiB) sit in the 256 MB Infinity Cache; each step is one launch "
-                     f"over {n} nodes, bound by latency, not by HBM",
+                     f"({nt * n * 8 / 2**20:.0f} MiB) sit on the chip or in the 256 MB Infinity Cache; "
+                     f"{n} nodes are bound by a step's latency, not by HBM",
     }
     if not args.no_cpu:
         cpu = cpu_gradient(solver, shot, 20.0)
@@ -788,7 +788,8 @@ def main():
     }
 
     if resident is not None:
-        result["roofline"].update(bound="vector instructions of the PML rows",
+        # neither memory nor one unit (counters, profiles/k_resident2d_layered2d_16shots.md)
+        result["roofline"].update(bound="latency of a step on the chip (vector instructions and waits of the PML rows)",
                                   kernel="k_resident2d<float,4,4> (adjoint + imaging, fields on the chip; per step)")
         result["forward_kernel"]["kernel"] = "k_resident2d<float,4,1> (forward + dWaveOp store, fields on the chip; " \
                                              "per step)"

@@ -7,9 +7,11 @@
 // Shots are independent and a shot's fields are small, so here a launch keeps
 // them in registers and LDS for hundreds of steps: only the forward history
 // (dWaveOp, written or read once per step), the receivers' nodes and the rows
-// at strip borders move.  Now 18.1 and 20.3 us for the 16 shots, 3.2 us for
-// the small one; bound by the vector instructions of the PML rows (6 times a
-// plain row's), with few strips by the exchange of border rows.
+// at strip borders move.  Now 17.3 and 19.8 us for the 16 shots, 3.0 us for
+// the small one.  With few strips the exchange of border rows bounds a step;
+// with many the waves of the PML rows, by their vector instructions (all SIMDs
+// together issue them in 57 % of the cycles) and their waits (56 % of a wave's
+// cycles; the LDS is busy in 18 %, bank conflicts 5 %).
 //
 // Split: a shot is cut along x into strips of whole rows, one 512-thread
 // workgroup per strip, one workgroup per CU.  u of the strip (and Phi where

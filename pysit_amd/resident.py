@@ -461,7 +461,8 @@ def thread_items(lay, xtype, nzc, zfl, zfr, R, limits):
 
 
 # a plan holds 0.1 to 0.6 MB; a survey of shots of uneven aperture,
-# modeled shot by shot, comes back to each of its plans (1.5 to 8 ms to make)
+# modeled shot by shot, comes back to each of its plans (4 ms to make, 9 to 14
+# those of 16 to 32 shots)
 _PLANS = _Kept(256)
 
 
